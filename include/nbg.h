@@ -83,9 +83,8 @@ typedef struct nbg_params {
     float eps2;          /* Gravity "epsilon", added to r^2; default 1e-5 (Gravity.h:195,207) */
     float dt;            /* Solver::timeStep(), default 1e-3 (Simulation/Solver.h:34,101) */
     int32_t sum_mode;    /* nbg_sum_mode */
-    int32_t targets_per_lane; /* FAST walks: bodies each lane walks the tree for, 1, 2 or 4 (0 reads as 1);
-                                 a wavefront serves 64 x this many bodies (no reference counterpart:
-                                 a schedule choice that leaves every result's interaction set unchanged) */
+    int32_t targets_per_lane; /* 1, 2 or 4 (0 reads as 1): a schedule hint for the FAST walks, which changes no
+                                 result and which the present walks do not need (no reference counterpart) */
 } nbg_params;
 
 typedef struct nbg_ctx nbg_ctx;
@@ -196,17 +195,15 @@ int nbg_sys_enable_counts(nbg_sys *sys, int32_t on);
 int nbg_sys_enable_walk_stats(nbg_sys *sys, int32_t on);
 int nbg_sys_walk_stats(nbg_sys *sys, uint64_t *out4);
 
-/* Waves per group of 64 targets in the tree walks (FAST: linear BVH with one
- * target per lane, octree; ORDERED: linear BVH; no reference counterpart: a
- * schedule choice).  0 (the default) chooses by size: systems of at most
- * 65,536 bodies fill the GPU with up to 16 waves per group, within 4,096
- * waves in all (FAST: linear BVH 4, octree 8), larger ones use 1.  Results are the same bits for every
- * choice: FAST sums each target's interactions per fixed block of subtrees and
- * adds the blocks in one order (the forest and the several-targets-per-lane
- * walks use the same blocks); ORDERED computes each frontier subtree's result
- * from zero, as the reference's recursion does, and adds it where the walk
- * meets it.  A split walk keeps 408 (FAST) or 1,536 (ORDERED) bytes per body
- * of sums in HBM. */
+/* Waves that share a group of targets in the tree walks (no reference
+ * counterpart: a schedule choice).  0 (the default) chooses by size: small
+ * systems fill the GPU with up to 4 waves per 16 targets (FAST) or, up to
+ * 65,536 bodies, 16 waves per 64 targets (ORDERED), within 4,096 waves in
+ * all; larger ones use 1.  Results are the same bits for every choice: FAST
+ * sums each target's interactions in four fixed classes, which the waves
+ * share out; ORDERED computes each frontier subtree's result from zero, as
+ * the reference's recursion does, and adds it where the walk meets it.  A
+ * split ORDERED walk keeps 1,536 bytes per body of results in HBM. */
 int nbg_sys_set_walk_split(nbg_sys *sys, int32_t waves);
 
 /* Per-phase device time (ms) of the last force pass, measured with HIP events
@@ -349,28 +346,24 @@ int nbg_batch_use_graph(nbg_batch *b, int32_t on);
 int nbg_batch_autotune(nbg_batch *b, const int32_t *leaf_sizes, int32_t k, int32_t repeats, int32_t *best,
                        float *ms_out);
 
-/* The autotuner over leaf size x bodies per wavefront: times every pair
- * (leaf_sizes[i], targets per lane tpls[j] in {1, 2, 4}; a wavefront serves
- * 64 x tpl bodies) as above and keeps the fastest pair.  ms_out[i * kt + j]
- * (optional) receives each mean pass time, -1 for pairs the batch's walk
- * does not run (more than one target per lane exists for the FAST
- * linear-BVH walk only).  The traversal stacks need no tuning: each walk's
- * stack holds the deepest path its trees can have. */
+/* The autotuner over leaf size x targets per lane: times every pair
+ * (leaf_sizes[i], tpls[j] in {1, 2, 4}) as above and keeps the fastest pair.
+ * ms_out[i * kt + j] (optional) receives each mean pass time, -1 for pairs
+ * the batch does not offer (more than one target per lane exists for FAST
+ * linear-BVH batches only, where it is a hint: see nbg_params).  The
+ * traversal stacks need no tuning: each walk's stack holds what its trees
+ * can need. */
 int nbg_batch_autotune_grid(nbg_batch *b, const int32_t *leaf_sizes, int32_t kl, const int32_t *tpls, int32_t kt,
                             int32_t repeats, int32_t *best_leaf, int32_t *best_tpl, float *ms_out);
 
-/* Targets per lane of the batch's FAST linear-BVH walk (1, 2 or 4); the
+/* The targets-per-lane hint of the batch (1, 2 or 4; nbg_params); the
  * autotuner sets it too.  Results do not depend on it. */
 int nbg_batch_set_targets_per_lane(nbg_batch *b, int32_t tpl);
 
-/* Waves per group of 64 targets in the batch's FAST walks (no reference
- * counterpart: a schedule choice, as nbg_sys_set_walk_split).  0 (the
- * default) chooses by size: a forest of at most 65,536 bodies in all, walked
- * with one target per lane and with at least half of its bodies in systems of
- * 4,096 bodies or more, splits each group over up to 4 waves (octree: 8);
- * 1 never splits.  Each member's results are the same bits for every
- * choice.  A FAST batch keeps 408 bytes per body, for up to 65,536 bodies,
- * of split sums in HBM. */
+/* Waves per 16 targets in the batch's FAST walks (no reference counterpart:
+ * a schedule choice, as nbg_sys_set_walk_split).  0 (the default) chooses by
+ * the number of target groups; otherwise as asked, at most 4.  Each member's
+ * results are the same bits for every choice. */
 int nbg_batch_set_walk_split(nbg_batch *b, int32_t waves);
 
 /* ---- serving: continuous batching over a forest ----

@@ -382,8 +382,8 @@ class System:
         _check(lib().nbg_sys_enable_walk_stats(self.handle, int(on)))
 
     def set_walk_split(self, waves: int = 0):
-        """Waves per group of 64 targets in the FAST linear-BVH walk (0:
-        chosen by size; results are the same bits for every choice)."""
+        """Waves that share a group of targets in the tree walks (0: chosen
+        by size; results are the same bits for every choice)."""
         _check(lib().nbg_sys_set_walk_split(self.handle, int(waves)))
 
     def walk_stats(self) -> dict:
@@ -544,9 +544,8 @@ class Batch:
         _check(lib().nbg_batch_set_targets_per_lane(self.handle, int(tpl)))
 
     def set_walk_split(self, waves: int = 0):
-        """Waves per group of 64 targets in the FAST walks: 0 by size (forests
-        of at most 65,536 bodies, at least half of them in systems of 4,096 or
-        more, split), 1 off, or 2, 4, 8, 16."""
+        """Waves per 16 targets in the FAST walks: 0 by size, 1 off, or 2, 4, 8
+        or 16 (above 4 reads as 4)."""
         _check(lib().nbg_batch_set_walk_split(self.handle, int(waves)))
 
     def autotune(self, leaf_sizes=(8, 16, 32, 64), repeats: int = 2):

@@ -86,12 +86,10 @@ struct nbg_sys {
     int64_t fmm_item_cap = 0, fmm_pool_cap = 0;
     int fmm_seed_cap = 0;
     int fmm_shift = 0;  // capacity doublings after passes that outgrew the pool
-    // split FAST linear-BVH walks of small systems: per-target sums and
-    // per-group block counts (see WalkArgs::split); split_req 0 = automatic
-    double *split_part = nullptr;
-    int32_t *split_nb = nullptr;
+    // split ORDERED walks of small systems: per-target results of the frontier
+    // subtrees (see WalkArgs::split); split_req 0 = automatic
+    float *split_part = nullptr;
     int64_t split_cap = 0;
-    int64_t split_words = 0;  // doubles per target in split_part
     int split_req = 0;
     // passive-point walks (nbg_sys_accelerations_at): one buffer that grows
     // to the largest target count seen and is kept for later calls
@@ -221,55 +219,34 @@ int ensure_fmm(nbg_sys *s) {
     return NBG_OK;
 }
 
-bool is_lbvh(int solver) { return solver == NBG_LINEAR_BVH || solver == NBG_LINEAR_BVH_QUADRUPOLE; }
-
-// Split waves per group for the system's tree walk (1 for the other
-// solvers and several targets per lane).  The FAST octree's frontier holds
-// at most 8 blocks, so it uses at most 8 waves; by size the FAST linear-BVH
-// walk uses at most 4 (measured fastest from 2,000 to 65,536 bodies).
+// Waves per group of targets in the system's tree walk (1 for the other
+// solvers): chosen by size, or as requested (FAST walks use at most 4).
 int split_of(const nbg_sys *s) {
-    const bool lbvh = is_lbvh(s->prm.solver);
-    const bool tree = lbvh || s->prm.solver == NBG_BARNES_HUT || s->prm.solver == NBG_BARNES_HUT_QUADRUPOLE;
-    if (s->prm.sum_mode != NBG_SUM_FAST) {
-        if (!tree || s->n > kOrderedSplitMaxBodies) return 1;
-        return s->split_req > 0 ? s->split_req : split_waves(s->n);
-    }
-    if (!lbvh && !(is_octree(s->prm.solver) && s->prm.solver != NBG_IMPLICIT_FMM)) return 1;
-    if (lbvh && s->prm.targets_per_lane > 1) return 1;
-    if (s->split_req > 0) return lbvh ? s->split_req : std::min(s->split_req, 8);
-    return std::min(split_waves(s->n), lbvh ? kSplitAutoLbvh : 8);
+    if (s->prm.solver == NBG_NAIVE || s->prm.solver == NBG_IMPLICIT_FMM) return 1;
+    if (s->prm.sum_mode == NBG_SUM_FAST)
+        return s->split_req > 0 ? std::min(s->split_req, 4) : fast_split_waves((s->n + 63) / 64);
+    if (s->n > kOrderedSplitMaxBodies) return 1;
+    return s->split_req > 0 ? s->split_req : ordered_split_waves(s->n);
 }
 
 void free_split(nbg_sys *s) {
     if (s->split_part) (void)hipFree(s->split_part);
-    if (s->split_nb) (void)hipFree(s->split_nb);
     s->split_part = nullptr;
-    s->split_nb = nullptr;
     s->split_cap = 0;
-    s->split_words = 0;
 }
 
-// Allocates the split walk's sums when the system's walk splits (no-op
-// otherwise or when the current ones are large enough).
-// Doubles of split sums per target: the FAST blocks' FP64 sums, or the
-// ORDERED frontier results (FP32, two to a double).
-int64_t split_words(const nbg_sys *s) {
-    return s->prm.sum_mode == NBG_SUM_FAST ? (int64_t)kSplitSlots * 3 : (int64_t)kOrderedSplitSlots * 3 / 2;
-}
-
+// Allocates the ORDERED split walk's results when the system's walk splits
+// (no-op otherwise or when the current ones are large enough).
 int ensure_split(nbg_sys *s) {
-    if (split_of(s) <= 1 || (s->split_cap >= s->n && s->split_words >= split_words(s))) return NBG_OK;
+    if (s->prm.sum_mode == NBG_SUM_FAST || split_of(s) <= 1 || s->split_cap >= s->n) return NBG_OK;
     if (s->stream) NBG_HIP(hipStreamSynchronize(s->stream));
     free_split(s);
     const int64_t n = s->n > 0 ? s->n : 1;
-    int r = dalloc(&s->split_part, split_words(s) * n);
-    if (r == NBG_OK) r = dalloc(&s->split_nb, (n + 63) / 64);
-    if (r != NBG_OK) {
+    if (int r = dalloc(&s->split_part, (int64_t)kOrderedSplitSlots * 3 * n)) {
         free_split(s);
         return r;
     }
     s->split_cap = n;
-    s->split_words = split_words(s);
     return NBG_OK;
 }
 
@@ -417,11 +394,11 @@ int enqueue_force_pass(nbg_sys *s) {
     } else {
         WalkArgs wa = walk_args(s);
         const int k = split_of(s);
-        if (k > 1 && s->split_part && s->split_cap >= s->n && s->split_words >= split_words(s)) {
+        if (p.sum_mode == NBG_SUM_FAST) {
             wa.split = k;
-            wa.split_part = s->split_part;
-            wa.split_part_f = reinterpret_cast<float *>(s->split_part);
-            wa.split_nb = s->split_nb;
+        } else if (k > 1 && s->split_part && s->split_cap >= s->n) {
+            wa.split = k;
+            wa.split_part_f = s->split_part;
             wa.split_stride = s->n;
         }
         const int stats = s->walk_stats ? 2 : (s->counting ? 1 : 0);
@@ -459,7 +436,6 @@ WalkArgs walk_args(nbg_sys *s) {
     wa.counts = s->counts();
     wa.err = s->err_word();
     wa.quad = is_quad(p.solver) ? s->quad : nullptr;
-    wa.tpl = p.targets_per_lane > 1 ? p.targets_per_lane : 1;
     return wa;
 }
 
@@ -635,6 +611,7 @@ int walk_points(nbg_sys *s, int64_t nt, const float *tx, const float *ty, const 
     launch_fill_u32(s->misc + 4, 0u, 12, st);
     WalkArgs wa = walk_args(s);
     wa.nt = nt;
+    if (s->prm.sum_mode == NBG_SUM_FAST) wa.split = fast_split_waves((nt + 63) / 64);
     wa.targets = pb.t4;
     wa.perm = pb.i2;
     wa.ax = pb.a3;

@@ -285,7 +285,7 @@ template <bool SOFT>
 __device__ void fmm_walk_from(const FmmArgs &a, const OctRec &st, uint64_t lanes, FastWave &W, int *s_grp,
                               uint64_t *s_msk, bool &fail) {
     const OctRec *__restrict__ nodes = a.nodes;
-    uint64_t mask = visit_oct<SOFT, 1, false>(st, nullptr, lanes, a.bodies, a.n, a.eps2, W, fail);
+    uint64_t mask = visit_oct<SOFT>(st, lanes, a.bodies, a.n, a.eps2, W, fail);
     int c = st.topo.z, nch = oct_nchild(st);
     int sp = 0;
     int64_t iters = 0;
@@ -309,7 +309,7 @@ __device__ void fmm_walk_from(const FmmArgs &a, const OctRec &st, uint64_t lanes
         int nc = 0, nn = 0;
         for (int k = 0; k < nch; ++k) {
             const OctRec r = nodes[c + k];
-            const uint64_t o = visit_oct<SOFT, 1, false>(r, nullptr, mask, a.bodies, a.n, a.eps2, W, fail);
+            const uint64_t o = visit_oct<SOFT>(r, mask, a.bodies, a.n, a.eps2, W, fail);
             if (o) {
                 if (nm) {
                     if (sp >= kStackOct) { fail = true; break; }

@@ -259,44 +259,35 @@ struct WalkArgs {
     // Quadrupole trees: second moments per node slot (2 float4, layout in
     // device.hpp); null for monopole trees.
     const float4 *quad = nullptr;
-    // FAST single-system walks: targets per lane (1, 2 or 4); a wavefront
-    // serves 64 tpl consecutive targets, lane l of slot t target 64 t + l.
-    int tpl = 1;
-    // FAST single-system linear-BVH walks with one target per lane: split
-    // waves per group of 64 targets (1 = none).  With split > 1 the walk
-    // stores per-target sums in split_part (kSplitSlots x 3 doubles per
-    // target, component-major, split_stride doubles apart) and per-group
-    // block counts in split_nb, and a second kernel adds them up.
+    // Small systems: waves that share a group of targets (1 = none).  FAST: 1,
+    // 2 or 4 waves per 16 targets.  ORDERED: waves per 64 targets, each storing
+    // its frontier subtrees' results in split_part_f (kOrderedSplitSlots x 3
+    // floats per target, split_stride floats apart) for a second kernel.
     int split = 1;
-    double *split_part = nullptr;
-    float *split_part_f = nullptr;  // ORDERED split: kMaxFrontier x 3 floats per target
-    int32_t *split_nb = nullptr;
+    float *split_part_f = nullptr;
     int64_t split_stride = 0;
 };
 
-// Sums a split walk stores per target: the top nodes' and one per block of
-// frontier subtrees.
-constexpr int kSplitSlots = 17;
-// Largest system whose FAST linear-BVH walk splits its groups over waves.
-constexpr int64_t kSplitMaxBodies = 65536;
-// Waves per group the FAST linear-BVH walk takes when chosen by size.
-constexpr int kSplitAutoLbvh = 4;
 // ORDERED split: one result per frontier subtree (at most kOrderedSplitSlots)
 // per target, for systems of at most kOrderedSplitMaxBodies bodies.
 constexpr int kOrderedSplitSlots = 128;
 constexpr int64_t kOrderedSplitMaxBodies = 65536;
-// Split waves per group for a walk of `groups` groups of 64 targets, and
-// for a system of n bodies (1: the chip is full): the most waves, up to 16
-// per group, that keep the launch within 4,096 waves (16 per CU; measured:
-// wider launches of the split walks run slower from 30k bodies up).
-inline int split_waves_groups(int64_t groups) {
+// ORDERED split waves per group for a system of n bodies (1: the chip is
+// full): the most waves, up to 16 per group, that keep the launch within
+// 4,096 waves (16 per CU; measured: wider launches of the split walks run
+// slower from 30k bodies up).
+inline int ordered_split_waves(int64_t n) {
+    if (n > kOrderedSplitMaxBodies || n < 1) return 1;
     int k = 1;
-    while (k < 16 && groups * k * 2 <= 4096) k *= 2;
+    while (k < 16 && (n + 63) / 64 * k * 2 <= 4096) k *= 2;
     return k;
 }
-inline int split_waves(int64_t n) {
-    if (n > kSplitMaxBodies || n < 1) return 1;
-    return split_waves_groups((n + 63) / 64);
+// FAST waves per 16 targets for a walk of `groups` groups of 64 targets: the
+// most, up to 4, that keep the launch within 4,096 waves (4 per SIMD).
+inline int fast_split_waves(int64_t groups) {
+    int k = 1;
+    while (k < 4 && groups * 4 * k * 2 <= 4096) k *= 2;
+    return k;
 }
 
 // Barnes-Hut traversal over the LBVH.  ordered != 0 selects the
@@ -306,6 +297,9 @@ void launch_walk_lbvh(const WalkArgs &a, int ordered, int max_depth, int diag, h
 
 // Barnes-Hut traversal over the octree (same modes and statistics).
 void launch_walk_oct(const WalkArgs &a, int ordered, int diag, hipStream_t s);
+
+// The FAST walks of both trees (walk_fast.hip).
+void launch_walk_fast(const WalkArgs &a, bool octree, int stats, hipStream_t s);
 
 // Implicit FMM (fmm.hip): the lockstep dual traversal breadth-first, one
 // launch per traversal step, then one launch for the passive leaves.
