@@ -153,7 +153,7 @@ int ensure_octree(nbg_sys *s) {
     A(&b.nown, n); A(&b.nbase, n);
     A(&b.nfirst, cap); A(&b.ncount, cap); A(&b.nparent, cap); A(&b.nmeta, cap);
     A(&b.occ, cap); A(&b.cb, cap); A(&b.flags, cap); A(&b.glist, 2 * (cap + 64));
-    A(&b.scan_ws, 128 + (cap + kScanTile - 1) / kScanTile);
+    A(&b.scan_ws, oct_scan_words(n, cap));
     A(&b.nodes, cap); A(&b.centre, cap); A(&b.thr, 64); A(&b.misc, 64);
     if (r != NBG_OK) {
         free_oct(b);
@@ -310,16 +310,18 @@ int enqueue_force_pass(nbg_sys *s) {
     const bool octree = is_octree(p.solver);
     if (int r = ensure_buffers(s)) return r;
     float4 *quad = is_quad(p.solver) ? s->quad : nullptr;
-    launch_fill_u32(s->misc + 4, 0u, 12, st);  // interaction counters
     if (p.solver == NBG_NAIVE) {
         // NaiveSolver: no tree; every body sums every body in body order.
         // SimpleTrackingRule counts n calls per body, np = 0.
         for (int k = 0; k <= 5; ++k) mark(s, k);
-        launch_fill_u32(s->node_count(), 0u, 1, st);
         launch_pack(s->x, s->y, s->z, s->m, n, s->bodies, st);
         const uint64_t pp = (uint64_t)n * (uint64_t)n;
-        launch_fill_u32(s->misc + 4, (uint32_t)pp, 1, st);
-        launch_fill_u32(s->misc + 5, (uint32_t)(pp >> 32), 1, st);
+        FillSet fills;
+        fills.add(s->node_count(), 1);
+        fills.add(s->misc + 4, 1, (uint32_t)pp);
+        fills.add(s->misc + 5, 1, (uint32_t)(pp >> 32));
+        fills.add(s->misc + 6, 10);
+        launch_fills(fills, st);
         mark(s, 6);
         launch_direct_f32(s->bodies, n, s->bodies, n, nullptr, p.G, p.eps2, p.sum_mode == NBG_SUM_ORDERED, s->ax,
                           s->ay, s->az, st);
@@ -329,32 +331,49 @@ int enqueue_force_pass(nbg_sys *s) {
         return NBG_OK;
     }
     mark(s, 0);
-    launch_bbox(s->x, s->y, s->z, n, s->bbox_partials, s->bbox, st);
+    // one launch clears what the build counts in
+    const int bits = octree ? 63 : p.morton_bits;
+    const bool lo = octree && oct_has_lo(p.max_depth);
+    const SortPlan plan = sort_plan(n, bits, lo);
+    FillSet fills;
+    fills.add(s->misc + 4, 12);  // interaction counters
+    if (n > 0) {
+        fills.add(s->sort_status, sort_clear_words(n, plan));
+        if (octree) oct_fills(fills, s->ob, n, s->leaf_start);
+        else lbvh_fills(fills, n, s->leaf_start, s->scan_ws, s->flags);
+    } else {
+        fills.add(s->bbox, 3, 0x7f7fffffu);      // the empty box: FLT_MAX, -FLT_MAX
+        fills.add(s->bbox + 3, 3, 0xff7fffffu);
+    }
+    const int parts = launch_bbox(s->x, s->y, s->z, n, s->bbox_partials, fills, st);
     mark(s, 1);
     if (octree) {
         OctBuffers &ob = s->ob;
         uint64_t *keys = (uint64_t *)s->keys, *keys_alt = (uint64_t *)s->keys_alt;
-        launch_octree_keys(s->x, s->y, s->z, n, s->bbox, p.max_depth, ob, keys, s->idx, s->idx_alt, st);
+        // sorted keys in keys, the key order in idx_alt's place: the leaves' order goes to idx
+        launch_octree_keys(s->x, s->y, s->z, n, s->bbox_partials, parts, s->bbox, p.max_depth, p.theta, plan, ob, keys,
+                           s->idx_alt, keys_alt, s->idx, s->sort_status, st);
         mark(s, 2);
-        launch_octree_sort(n, p.max_depth, ob, keys, s->idx, keys_alt, s->idx_alt, s->sort_status, s->err_word(), st);
+        launch_sort(keys, s->idx_alt, keys_alt, s->idx, n, bits, plan, s->sort_status, s->err_word(), st,
+                    lo ? ob.key_lo : nullptr, ob.lo_sorted);
         mark(s, 3);
-        launch_octree_topology(n, s->bbox, p.leaf_size, p.max_depth, p.theta, ob, keys, s->idx_alt, s->idx,
-                               s->leaf_start, s->err_word(), st);
+        launch_octree_topology(n, s->bbox, p.leaf_size, p.max_depth, ob, keys, s->idx_alt, s->idx, s->leaf_start,
+                               s->err_word(), st);
         mark(s, 4);
         launch_gather(s->x, s->y, s->z, s->m, s->idx, n, s->bodies, st);
         mark(s, 5);
         launch_octree_summaries(s->bodies, n, ob, s->leaf_start, s->err_word(), st, quad);
     } else {
-        launch_morton(s->x, s->y, s->z, n, s->bbox, p.morton_bits, s->keys, s->idx, st);
+        launch_morton(s->x, s->y, s->z, n, s->bbox_partials, parts, s->bbox, bits, plan, s->keys, s->idx, s->keys_alt,
+                      s->idx_alt, s->sort_status, st);
         mark(s, 2);
-        launch_radix_sort(s->keys, s->idx, s->keys_alt, s->idx_alt, n, p.morton_bits, s->sort_status, s->err_word(),
-                          st);
+        launch_sort(s->keys, s->idx, s->keys_alt, s->idx_alt, n, bits, plan, s->sort_status, s->err_word(), st);
         mark(s, 3);
-        launch_lbvh_topology(s->keys, p.morton_bits, n, p.leaf_size, s->kfirst, s->klast, s->kgamma, s->ksplit,
-                             s->krank, s->kparent, s->scan_ws, s->nodes, s->leaf_start, s->node_count(), st);
+        launch_lbvh_topology(s->keys, bits, n, p.leaf_size, s->kfirst, s->klast, s->kgamma, s->ksplit, s->krank,
+                             s->kparent, s->scan_ws, s->nodes, s->leaf_start, s->node_count(), s->x, s->y, s->z, s->m,
+                             s->idx, s->bodies, st);
         mark(s, 4);
-        launch_gather(s->x, s->y, s->z, s->m, s->idx, n, s->bodies, st);
-        mark(s, 5);
+        mark(s, 5);  // the bodies are gathered with the topology
         launch_lbvh_summaries(s->bodies, n, s->nodes, s->leaf_start, 2 * n, s->flags, s->glist, s->bmin, s->bmax,
                               p.theta, s->err_word(), st, nullptr, nullptr, 0, quad);
     }
@@ -605,10 +624,15 @@ int walk_points(nbg_sys *s, int64_t nt, const float *tx, const float *ty, const 
     NBG_HIP(hipMemcpyAsync(pb.t3, tx, b, hipMemcpyHostToDevice, st));
     NBG_HIP(hipMemcpyAsync(pb.t3 + nt, ty, b, hipMemcpyHostToDevice, st));
     NBG_HIP(hipMemcpyAsync(pb.t3 + 2 * nt, tz, b, hipMemcpyHostToDevice, st));
-    launch_morton(pb.t3, pb.t3 + nt, pb.t3 + 2 * nt, nt, s->bbox, 63, pb.k2, pb.i2, st);
-    launch_radix_sort(pb.k2, pb.i2, pb.k2 + nt, pb.i2 + nt, nt, 63, pb.status, s->err_word(), st);
+    const SortPlan plan = sort_plan(nt, 63, false);
+    FillSet fills;
+    fills.add(pb.status, sort_clear_words(nt, plan));
+    fills.add(s->misc + 4, 12);
+    launch_fills(fills, st);
+    launch_morton(pb.t3, pb.t3 + nt, pb.t3 + 2 * nt, nt, nullptr, 0, s->bbox, 63, plan, pb.k2, pb.i2, pb.k2 + nt,
+                  pb.i2 + nt, pb.status, st);
+    launch_sort(pb.k2, pb.i2, pb.k2 + nt, pb.i2 + nt, nt, 63, plan, pb.status, s->err_word(), st);
     launch_gather(pb.t3, pb.t3 + nt, pb.t3 + 2 * nt, pb.t3, pb.i2, nt, pb.t4, st);
-    launch_fill_u32(s->misc + 4, 0u, 12, st);
     WalkArgs wa = walk_args(s);
     wa.nt = nt;
     if (s->prm.sum_mode == NBG_SUM_FAST) wa.split = fast_split_waves((nt + 63) / 64);

@@ -226,7 +226,7 @@ int ensure_octree(nbg_batch *b) {
         A(&o.key_hi, n); A(&o.key_lo, n); A(&o.lo_sorted, n); A(&o.nown, n); A(&o.nbase, n);
         A(&o.nfirst, cap); A(&o.ncount, cap); A(&o.nparent, cap); A(&o.nmeta, cap);
         A(&o.occ, cap); A(&o.cb, cap); A(&o.flags, cap); A(&o.glist, 2 * (cap + 64));
-        A(&o.scan_ws, 128 + (cap + kScanTile - 1) / kScanTile);
+        A(&o.scan_ws, oct_scan_words(n, cap));
         A(&o.nodes, cap); A(&o.centre, cap); A(&o.thr, (int64_t)kOctThrStride * b->cap_s); A(&o.misc, 64);
         if (r != NBG_OK) {
             free_octree(o);
@@ -302,6 +302,10 @@ void enqueue_pass_octree(nbg_batch *b) {
     const int S = (int)b->sys.size();
     hipStream_t s = b->stream;
     OctBuffers &ob = b->ob;
+    FillSet fills;
+    oct_fills(fills, ob, n, b->leaf_start);
+    fills.add(b->misc + 4, 12);
+    launch_fills(fills, s);
     launch_seg_bbox(b->x(), b->y(), b->z(), S, b->sys_first, b->bbox6, s);
     launch_octree_forest_build(b->x(), b->y(), b->z(), n, S, b->bsys, b->bbox6, b->lv_tab, b->max_levels, ob,
                                b->keys, b->idx, b->keys_alt, b->idx_alt, b->sort_status, b->err_word(), s);
@@ -348,17 +352,22 @@ void enqueue_pass(nbg_batch *b) {
     const int64_t n = b->n;
     const int S = (int)b->sys.size();
     hipStream_t s = b->stream;
-    launch_fill_u32(b->misc + 4, 0u, 12, s);
-    if (n == 0) return;
+    if (n == 0) {
+        launch_fill_u32(b->misc + 4, 0u, 12, s);
+        return;
+    }
     if (is_octree_solver(b->solver)) {
         enqueue_pass_octree(b);
         return;
     }
+    FillSet fills;
+    lbvh_fills(fills, n, b->leaf_start, b->scan_ws, b->flags);
+    fills.add(b->misc + 4, 12);
     launch_forest_build(b->x(), b->y(), b->z(), n, S, b->sys_first, b->bsys, b->bbox6, b->keys, b->idx, b->keys_alt,
-                        b->idx_alt, b->sort_status, b->err_word(), s);
+                        b->idx_alt, b->sort_status, fills, b->err_word(), s);
     launch_lbvh_topology(b->keys, 63, n, 0, b->kfirst, b->klast, b->kgamma, b->ksplit, b->krank, b->kparent,
-                         b->scan_ws, b->nodes, b->leaf_start, b->node_count(), s, 30, b->leaf_tab);
-    launch_gather(b->x(), b->y(), b->z(), b->m(), b->idx, n, b->bodies, s);
+                         b->scan_ws, b->nodes, b->leaf_start, b->node_count(), b->x(), b->y(), b->z(), b->m(), b->idx,
+                         b->bodies, s, 30, b->leaf_tab);
     float4 *quad = b->solver == NBG_LINEAR_BVH_QUADRUPOLE ? b->quad : nullptr;
     launch_lbvh_summaries(b->bodies, n, b->nodes, b->leaf_start, 2 * n, b->flags, b->glist, b->bmin, b->bmax, 0.5f,
                           b->err_word(), s, b->mp_tab, b->keys, 30, quad);

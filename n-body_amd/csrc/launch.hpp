@@ -7,23 +7,81 @@
 
 namespace nbg {
 
-// Radix-sort geometry (onesweep): 256 threads x 16 keys per tile.
+// Radix-sort geometry (onesweep): 256 threads x kSortItems keys per tile.
+// Fewer keys a thread while more would leave the chip short of tiles: a pass
+// over u64 keys takes 6.7 us with 4 keys a thread and 11.0 with 16 at 10,000
+// keys, 16.8 with 8 and 18 with 16 at 500,000, 27 with 8 and 23 with 16 at
+// 1,048,576.
 constexpr int kSortBlock = 256;
-constexpr int kSortItems = 16;
-constexpr int kSortTile = kSortBlock * kSortItems;
+constexpr int64_t kSortSmall = (int64_t)1 << 18, kSortMedium = (int64_t)1 << 19;
+constexpr int sort_items(int64_t n) { return n <= kSortSmall ? 4 : n <= kSortMedium ? 8 : 16; }
 constexpr int kRadix = 256;
 
-constexpr int64_t sort_tiles(int64_t n) { return (n + kSortTile - 1) / kSortTile; }
+constexpr int64_t sort_tiles(int64_t n) {
+    const int64_t tile = (int64_t)kSortBlock * sort_items(n);
+    return (n + tile - 1) / tile;
+}
+// The most tiles of any n' <= n (a smaller sort may use smaller tiles).
+constexpr int64_t sort_tiles_upto(int64_t n) {
+    int64_t t = sort_tiles(n);
+    if (n > kSortSmall && sort_tiles(kSortSmall) > t) t = sort_tiles(kSortSmall);
+    if (n > kSortMedium && sort_tiles(kSortMedium) > t) t = sort_tiles(kSortMedium);
+    return t;
+}
 constexpr int sort_passes(int key_bits) { return (key_bits + 7) / 8; }
-// Words of status memory one sort needs (per pass: tiles x 256 + counters).
+// Words of status memory one sort needs: histograms, tile counters, the list
+// of long runs, and per pass the tiles' look-back words.
+constexpr int kSortLongRuns = 4096;
+constexpr int64_t kSortHeadWords = 8 * kRadix + 64 + 2 * kSortLongRuns;
 constexpr int64_t sort_status_words(int64_t n, int key_bits) {
-    return 8 * kRadix + 64 + (int64_t)sort_passes(key_bits) * (sort_tiles(n) * kRadix);
+    return kSortHeadWords + (int64_t)sort_passes(key_bits) * (sort_tiles_upto(n) * kRadix);
+}
+
+// How n keys of `bits` significant bits are sorted: `passes` radix passes over
+// the bits from `shift` up, from the _alt buffers if from_alt, then (runs) the
+// runs of keys that share those bits put in order.  Results land in the
+// primary buffers.  lo: the keys have a low word too.
+struct SortPlan {
+    int passes, shift;
+    bool runs, from_alt;
+};
+inline SortPlan sort_plan(int64_t n, int bits, bool lo) {
+    const int full = sort_passes(bits);
+    int need = 10;  // log2 n + 10 bits tell most bodies' spatial keys apart
+    while (((int64_t)1 << (need - 10)) < n) ++need;
+    SortPlan p;
+    p.passes = sort_passes(need) < full ? sort_passes(need) : full;
+    p.shift = bits > 8 * p.passes ? bits - 8 * p.passes : 0;
+    p.runs = p.shift > 0 || lo;
+    // the last kernel reads the _alt buffers (runs), or the last pass writes the primary ones
+    p.from_alt = p.runs ? (p.passes & 1) == 0 : (p.passes & 1) != 0;
+    return p;
+}
+// Words of status memory that a planned sort of n keys uses (to be cleared first).
+inline int64_t sort_clear_words(int64_t n, const SortPlan &p) {
+    return kSortHeadWords + (int64_t)p.passes * sort_tiles(n) * kRadix;
 }
 
 // Scan geometry.
 constexpr int kScanBlock = 256;
 constexpr int kScanItems = 16;
 constexpr int kScanTile = kScanBlock * kScanItems;
+
+// Ranges of words that a build sets before its first use of them, in one
+// launch instead of one each.
+struct FillSet {
+    struct Range {
+        uint32_t *p;
+        int64_t n;
+        uint32_t v;
+    };
+    Range r[10];
+    int k = 0;
+    void add(void *p, int64_t n, uint32_t v = 0u) {
+        if (n > 0 && k < 10) r[k++] = Range{(uint32_t *)p, n, v};
+    }
+};
+void launch_fills(const FillSet &f, hipStream_t s);
 
 // Body count above which the tree arrays' 32-bit indices would overflow.
 constexpr int64_t kMaxBodies = (int64_t)1 << 29;
@@ -87,28 +145,49 @@ struct OctBuffers {
     uint32_t *cb = nullptr;        // cap: child counts, then their exclusive scan
     uint32_t *flags = nullptr;     // cap: summary arrival counters
     uint32_t *glist = nullptr;     // 2 * (cap + 64): two queues of straddling parents (summaries)
-    uint32_t *scan_ws = nullptr;   // 128 + cap / kScanTile
+    uint32_t *scan_ws = nullptr;   // the scan tiles' sums of nown, then of cb (oct_scan_words)
     OctRec *nodes = nullptr;       // cap, by slot
     float4 *centre = nullptr;      // cap, by slot: cell centre xyz, side
     float *thr = nullptr;          // 64: opening threshold per level
     uint32_t *misc = nullptr;      // 64: [0] node total, [1] child total
+    uint32_t *sums_own() const { return scan_ws; }
+    uint32_t *sums_child() const { return scan_ws + (n + kScanTile - 1) / kScanTile; }
 };
+inline int64_t oct_scan_words(int64_t n, int64_t cap) {
+    return (n + kScanTile - 1) / kScanTile + (cap + kScanTile - 1) / kScanTile + 1;
+}
+// What an octree build of n bodies counts in, to be set before it.
+inline void oct_fills(FillSet &f, const OctBuffers &ob, int64_t n, int32_t *leaf_start) {
+    f.add(ob.scan_ws, oct_scan_words(ob.n, ob.cap));
+    f.add(ob.occ, ob.cap);
+    f.add(leaf_start, n, 0xFFFFFFFFu);
+    f.add(ob.flags, ob.cap);
+    f.add(ob.glist, 64);
+    f.add(ob.glist + ob.cap + 64, 64);
+}
+// What a linear-BVH build of n bodies counts in, to be set before it.
+inline void lbvh_fills(FillSet &f, int64_t n, int32_t *leaf_start, uint32_t *scan_ws, uint32_t *flags) {
+    f.add(scan_ws, 64 + (n + kScanTile - 1) / kScanTile);
+    f.add(leaf_start, n, 0xFFFFFFFFu);
+    f.add(flags, 2 * n);
+}
 
 // Octree build (Octree::build, Trees/Octree.h:185-205) in three stages, each
-// enqueue-only.  keys: per-body octant path on the reference's float centre
-// recurrence.  sort: stable LSD radix sort by path (ties by original index);
-// idx_alt receives the key order.  topology: cells from the sorted keys,
-// node records, leaf contents reordered by original index into idx (the
-// final body order), leaf_start.  Summaries run after the body gather.
-void launch_octree_keys(const float *x, const float *y, const float *z, int64_t n, const float *bbox6,
-                        int max_depth, OctBuffers &ob, uint64_t *keys, uint32_t *idx, uint32_t *idx_alt,
-                        hipStream_t s);
-void launch_octree_sort(int64_t n, int max_depth, OctBuffers &ob, uint64_t *keys, uint32_t *idx,
-                        uint64_t *keys_alt, uint32_t *idx_alt, uint32_t *sort_status, uint32_t *err,
-                        hipStream_t s);
-void launch_octree_topology(int64_t n, const float *bbox6, int leaf_size, int max_depth, float theta,
-                            OctBuffers &ob, const uint64_t *keys, const uint32_t *idx_alt, uint32_t *idx,
-                            int32_t *leaf_start, uint32_t *err, hipStream_t s);
+// enqueue-only, after launch_bbox with oct_fills and the sort's words.
+// keys: per-body octant path on the reference's float centre recurrence (the
+// high word to the buffers that `plan` starts from, the low word to
+// ob.key_lo) and the levels' opening thresholds.  sort: launch_sort with
+// ob.key_lo / ob.lo_sorted when there is a low word.  topology: cells from
+// the sorted keys, node records, leaf contents reordered by original index
+// into idx (the final body order; idx_in is the key order), leaf_start.
+// Summaries run after the body gather.
+inline bool oct_has_lo(int max_depth) { return max_depth + 2 > kOctHiLevels; }
+void launch_octree_keys(const float *x, const float *y, const float *z, int64_t n, const float *partials, int blocks,
+                        float *bbox6, int max_depth, float theta, const SortPlan &plan, OctBuffers &ob, uint64_t *keys,
+                        uint32_t *idx, uint64_t *keys_alt, uint32_t *idx_alt, uint32_t *status, hipStream_t s);
+void launch_octree_topology(int64_t n, const float *bbox6, int leaf_size, int max_depth, OctBuffers &ob,
+                            const uint64_t *keys, const uint32_t *idx_in, uint32_t *idx, int32_t *leaf_start,
+                            uint32_t *err, hipStream_t s);
 // Forest of octrees: bodies of system s (bsys, original order) get paths
 // over their own system's cube (bbox6 + 6 s) and depth (lv_tab[s] levels);
 // the sort orders positions by system, then path.  Leaves the sorted high
@@ -137,53 +216,68 @@ void launch_octree_summaries(const float4 *bodies, int64_t n, OctBuffers &ob, co
 
 void launch_fill_u32(uint32_t *p, uint32_t v, int64_t n, hipStream_t s);
 
-// Exclusive scan of n u32 values into out (in may equal out); total (if not
-// null) receives the sum.  ws holds 64 + ceil(n / kScanTile) words.
-void launch_scan_u32(const uint32_t *in, uint32_t *out, int64_t n, uint32_t *ws, uint32_t *total, hipStream_t s);
+// Exclusive scan of n > 0 u32 values into out (in may equal out) from the
+// tiles' sums (ceil(n / kScanTile) words, overwritten); total receives the
+// sum.  nlim (or null): a device count of items, those past it being zero.
+// Up to kScanFused items the kernel that computes them adds up the tiles'
+// sums (one launch less; measured: 4 us less at 10,000 items, 20 us more at
+// 1,048,576, where the waves' atomics meet).
+constexpr int kScanFold = 4096;
+constexpr int64_t kScanFused = (int64_t)1 << 18;
+inline bool scan_fused(int64_t n) { return n <= kScanFused; }
+void launch_scan_u32(const uint32_t *in, uint32_t *out, int64_t n, uint32_t *sums, uint32_t *total, hipStream_t s,
+                     const uint32_t *nlim = nullptr);
 
 // Stable radix sort of u64 keys + u32 payload over the low 8 * passes bits.
 // Returns true when the result is in the _alt buffers (odd passes).
 bool launch_radix_sort_u64(uint64_t *keys, uint32_t *idx, uint64_t *keys_alt, uint32_t *idx_alt, int64_t n,
                            int passes, uint32_t *status, uint32_t *err, hipStream_t s);
 
-// outerBoundingBox: writes min xyz, max xyz to out6.  partials holds
-// 6 * kBBoxBlocks floats.
+// outerBoundingBox, first stage: per-block partials (6 * kBBoxBlocks floats),
+// and the ranges in `fills` set.  Returns the number of partials; the kernel
+// that computes the keys folds them and stores the box.
 constexpr int kBBoxBlocks = 512;
-void launch_bbox(const float *x, const float *y, const float *z, int64_t n, float *partials, float *out6,
-                 hipStream_t s);
+int launch_bbox(const float *x, const float *y, const float *z, int64_t n, float *partials, const FillSet &fills,
+                hipStream_t s);
 
-// Morton keys (bits = 30 -> u32 keys, 63 -> u64 keys) and iota payload.
-void launch_morton(const float *x, const float *y, const float *z, int64_t n, const float *bbox6, int bits,
-                   void *keys, uint32_t *idx, hipStream_t s);
+// Morton keys (bits = 30 -> u32 keys, 63 -> u64 keys) and iota payload into
+// the buffers that `plan` starts from, with the sort's histograms in `status`
+// (cleared).  blocks > 0: the box is folded from that many partials and
+// stored in bbox6; 0: bbox6 holds it.
+void launch_morton(const float *x, const float *y, const float *z, int64_t n, const float *partials, int blocks,
+                   float *bbox6, int bits, const SortPlan &plan, void *keys, uint32_t *idx, void *keys_alt,
+                   uint32_t *idx_alt, uint32_t *status, hipStream_t s);
 
-// Stable LSD radix sort of (key, idx) with onesweep passes.  Result lands
-// back in keys/idx (an even number of passes).  status must hold
-// sort_status_words(n, bits) words; err is a device flag word.
-void launch_radix_sort(void *keys, uint32_t *idx, void *keys_alt, uint32_t *idx_alt, int64_t n, int bits,
-                       uint32_t *status, uint32_t *err, hipStream_t s);
+// Stable sort of (key, idx) as planned (keys in place, status cleared and
+// with the histograms).  The result is in keys / idx.  lo (u64 keys): the
+// keys' low words by original index, lo_sorted receives them in key order.
+// err is a device flag word.
+void launch_sort(void *keys, uint32_t *idx, void *keys_alt, uint32_t *idx_alt, int64_t n, int bits,
+                 const SortPlan &plan, uint32_t *status, uint32_t *err, hipStream_t s, const uint64_t *lo = nullptr,
+                 uint64_t *lo_sorted = nullptr);
 
 // Sorted SoA -> float4 (x, y, z, m) in sort order.
 void launch_gather(const float *x, const float *y, const float *z, const float *m, const uint32_t *perm,
                    int64_t n, float4 *bodies, hipStream_t s);
 
 // LBVH topology (Karras radix tree truncated at the reference's leaf rule)
-// into the compact node arrays.  scratch ints: first,last,gamma,split,rank,
-// parent (6 * n words) plus scan_ws (sort_tiles-sized block sums + 64).
-// node_count receives the number of nodes.
+// into the compact node arrays, and the bodies in key order (perm).  scratch
+// ints: first, last, gamma, split, rank, parent (6 * n words) plus scan_ws
+// (64 words and the scan tiles' sums, cleared); leaf_start is set to -1
+// before.  node_count receives the number of nodes.
 void launch_lbvh_topology(const void *keys, int bits, int64_t n, int leaf_size, int32_t *kfirst,
                           int32_t *klast, int32_t *kgamma, uint32_t *ksplit, uint32_t *krank,
                           int32_t *kparent, uint32_t *scan_ws, NodeRec *nodes, int32_t *leaf_start,
-                          uint32_t *node_count, hipStream_t s, int sys_shift = 0,
+                          uint32_t *node_count, const float *x, const float *y, const float *z, const float *m,
+                          const uint32_t *perm, float4 *bodies, hipStream_t s, int sys_shift = 0,
                           const int32_t *leaf_tab = nullptr);
 
 // Bottom-up LBVH summaries with atomic arrival flags: COM, mass, bbox and the
 // MAC record (bbox centre, squared diagonal).  leaf_start[i] holds the leaf
 // slot whose first body is i (else -1; written by the topology pass);
-// flags holds max_nodes words; glist holds 2 * (2n + 64) words (two queues).
-constexpr int kSummBodies = 4096;   // bodies per workgroup in the local pass
-constexpr int kSummMidBodies = kSummBodies * 64;  // bodies per workgroup in the middle pass
-constexpr unsigned kSummMidMinBlocks = 8;         // fewer middle workgroups: no middle pass
-constexpr int kSummThreads = 1024;  // threads per workgroup in the local pass (latency hiding)
+// flags holds max_nodes words; glist holds 2 * (2n + 64) words (two queues
+// and their counts).
+constexpr int kSummBodies = 512;   // bodies per workgroup in the local pass, one per thread
 struct MacParam {       // mac_threshold's output for one theta
     double mid;
     int tie;
@@ -197,10 +291,12 @@ void launch_lbvh_summaries(const float4 *bodies, int64_t n, NodeRec *nodes, cons
                            const uint64_t *keys = nullptr, int sys_shift = 0, float4 *quad = nullptr);
 
 // Forest of independent systems (30-bit codes, u64 keys = system << 30 | code):
-// per-system bounding boxes (bbox6: 6 floats per system), keys, and one sort.
+// per-system bounding boxes (bbox6: 6 floats per system), keys, and one sort;
+// sets `fills` and the sort's words first.
 void launch_forest_build(const float *x, const float *y, const float *z, int64_t n, int nsys,
                          const int64_t *sys_first, const uint32_t *bsys, float *bbox6, uint64_t *keys, uint32_t *idx,
-                         uint64_t *keys_alt, uint32_t *idx_alt, uint32_t *sort_status, uint32_t *err, hipStream_t s);
+                         uint64_t *keys_alt, uint32_t *idx_alt, uint32_t *sort_status, FillSet &fills, uint32_t *err,
+                         hipStream_t s);
 // sys_root[s] = slot of the node whose range is exactly system s.
 void launch_forest_roots(const NodeRec *nodes, const uint32_t *node_count, int64_t max_nodes, const uint64_t *keys,
                          int64_t n, int nsys, int32_t *sys_root, uint32_t *err, hipStream_t s);

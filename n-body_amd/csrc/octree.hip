@@ -22,6 +22,7 @@
 // index, the order the reference's partitions leave them in when they are
 // stable.
 
+#include "build_common.hpp"
 #include "device.hpp"
 #include "launch.hpp"
 
@@ -185,6 +186,14 @@ __device__ float oct_threshold(float side, float theta) {
     return __uint_as_float(lo);
 }
 
+// The opening threshold of level L of the cube of bbox bb.
+__device__ float oct_level_threshold(const float *bb, int L, float theta) {
+    float cx, cy, cz, side;
+    oct_root(bb, cx, cy, cz, side);
+    for (int l = 0; l < L; ++l) side = side / 2.0f;
+    return oct_threshold(side, theta);
+}
+
 // ------------------------------------------------------------------ kernels
 
 // The octant path of a point over `levels` levels of the cube of bbox bb.
@@ -208,21 +217,31 @@ __device__ __forceinline__ void oct_path(const float *bb, int levels, float px, 
     }
 }
 
+// Keys, iota payload, the sort's digit histograms of the high word and (first
+// workgroup) the opening thresholds; the box is folded from k_bbox's partials.
 template <bool LO>
 __global__ __launch_bounds__(256) void k_oct_keys(const float *__restrict__ x, const float *__restrict__ y,
                                                   const float *__restrict__ z, int64_t n,
-                                                  const float *__restrict__ bb, int levels, uint64_t *khi,
-                                                  uint64_t *klo, uint64_t *klo_copy, uint32_t *idx) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    uint64_t hi, lo;
-    oct_path(bb, levels, x[i], y[i], z[i], hi, lo);
-    khi[i] = hi;
-    if (LO) {
-        klo[i] = lo;
-        klo_copy[i] = lo;
+                                                  const float *__restrict__ partials, int blocks, float *bbox6,
+                                                  int levels, float theta, float *thr, uint64_t *khi, uint64_t *klo,
+                                                  uint32_t *idx, uint32_t *ghist, int passes, int shift) {
+    __shared__ uint32_t h[8 * kRadix];
+    const DigitCount dc{h, passes, shift};
+    dc.clear();
+    float bb[6];
+    fold_bbox(partials, blocks, bb, bbox6);
+    __syncthreads();
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+        uint64_t hi, lo;
+        oct_path(bb, levels, x[i], y[i], z[i], hi, lo);
+        khi[i] = hi;
+        if (LO) klo[i] = lo;
+        idx[i] = (uint32_t)i;
+        dc.add(hi);
     }
-    idx[i] = (uint32_t)i;
+    __syncthreads();
+    dc.store(ghist);
+    if (blockIdx.x == gridDim.x - 1 && (int)threadIdx.x <= levels) thr[threadIdx.x] = oct_level_threshold(bb, threadIdx.x, theta);
 }
 
 __global__ __launch_bounds__(256) void k_gather_u64(const uint64_t *__restrict__ src,
@@ -265,12 +284,13 @@ __global__ __launch_bounds__(256) void k_gather_sys(const uint32_t *__restrict__
     dst[i] = j < n ? (uint64_t)bsys[j] : ~0ull;
 }
 
-__global__ __launch_bounds__(256) void k_oct_count(OctKeys K, int leaf, uint32_t *nown) {
+__global__ __launch_bounds__(256) void k_oct_count(OctKeys K, int leaf, uint32_t *nown, uint32_t *sums) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= K.n) return;
     uint32_t c = 0;
     oct_chain(K, i, leaf, [&](int, int64_t, bool) { ++c; });
     nown[i] = c;
+    scan_sum(c, i, sums);
 }
 
 __global__ __launch_bounds__(256) void k_oct_nodes(OctKeys K, int leaf, const uint32_t *__restrict__ nbase,
@@ -310,20 +330,12 @@ __global__ __launch_bounds__(256) void k_oct_nodes(OctKeys K, int leaf, const ui
 
 __global__ __launch_bounds__(256) void k_oct_nchild(const uint32_t *__restrict__ misc, int64_t cap,
                                                     const uint32_t *__restrict__ nmeta,
-                                                    const uint32_t *__restrict__ occ, uint32_t *nch) {
+                                                    const uint32_t *__restrict__ occ, uint32_t *nch, uint32_t *sums) {
     const int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (id >= cap) return;
-    const int64_t T = misc[0];
-    nch[id] = (id < T && !((nmeta[id] >> 12) & 1u)) ? (uint32_t)__popc(occ[id]) : 0u;
-}
-
-__global__ void k_oct_levels(const float *__restrict__ bb, int levels, float theta, float *thr) {
-    const int L = threadIdx.x;
-    if (L > levels) return;
-    float cx, cy, cz, side;
-    oct_root(bb, cx, cy, cz, side);
-    for (int l = 0; l < L; ++l) side = side / 2.0f;
-    thr[L] = oct_threshold(side, theta);
+    if (id >= cap || id >= (int64_t)misc[0]) return;
+    const uint32_t c = ((nmeta[id] >> 12) & 1u) ? 0u : (uint32_t)__popc(occ[id]);
+    nch[id] = c;
+    scan_sum(c, id, sums);
 }
 
 // Forest: block s computes system s's table (thr + kOctThrStride s) from
@@ -332,10 +344,7 @@ __global__ void k_oct_levels_forest(const float *__restrict__ bbox6, const int32
                                     const float4 *__restrict__ sys_prm, float *thr) {
     const int sy = blockIdx.x, L = threadIdx.x;
     if (L > lv_tab[sy]) return;
-    float cx, cy, cz, side;
-    oct_root(bbox6 + 6 * sy, cx, cy, cz, side);
-    for (int l = 0; l < L; ++l) side = side / 2.0f;
-    thr[kOctThrStride * sy + L] = oct_threshold(side, sys_prm[sy].z);
+    thr[kOctThrStride * sy + L] = oct_level_threshold(bbox6 + 6 * sy, L, sys_prm[sy].z);
 }
 
 // Slot of node id of system sy: a root takes slot sy (the roots of the
@@ -435,9 +444,13 @@ __global__ __launch_bounds__(256) void k_oct_leafsort(int64_t n, const int32_t *
 // (Tree::summarizeTreeTop, Trees/Tree.h:196-216), giving 0/0 = NaN there and
 // so a NaN root COM whenever a level-1 octant is empty.
 //
-// Scheduling as for the LBVH: workgroups own kSummBodies consecutive bodies,
+// Scheduling as for the LBVH: workgroups own kOctSummBodies consecutive bodies,
 // climb with workgroup-scope arrival counters while the parent's range stays
 // inside, and queue straddling parents for one final workgroup.
+
+constexpr int kOctSummBodies = 1024;                // bodies per workgroup in the local pass, one per thread
+constexpr int kOctSummMid = kOctSummBodies * 64;    // bodies per workgroup in the middle pass
+constexpr unsigned kOctSummMidMinBlocks = 8;        // fewer middle workgroups: no middle pass
 
 __device__ __forceinline__ uint32_t arrive(uint32_t *flag) {
     return __hip_atomic_fetch_add(flag, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -446,13 +459,19 @@ __device__ __forceinline__ uint32_t arrive(uint32_t *flag) {
 __device__ __forceinline__ void oct_summ_leaf(int s, int4 t, const float4 *__restrict__ bodies, OctRec *nodes,
                                               float4 *quad) {
     float M = 0.0f, cx = 0.0f, cy = 0.0f, cz = 0.0f;
-    for (int i = t.x; i < t.x + t.y; ++i) {
-        const float4 b = bodies[i];
+    auto add = [&](float4 b) {
         M += b.w;
         cx = cx + b.x * b.w;
         cy = cy + b.y * b.w;
         cz = cz + b.z * b.w;
+    };
+    // four loads in flight; the sums stay sequential
+    int i = t.x;
+    for (; i + 4 <= t.x + t.y; i += 4) {
+        const float4 b0 = bodies[i], b1 = bodies[i + 1], b2 = bodies[i + 2], b3 = bodies[i + 3];
+        add(b0); add(b1); add(b2); add(b3);
     }
+    for (; i < t.x + t.y; ++i) add(bodies[i]);
     nodes[s].com = make_float4(ieee_div(cx, M), ieee_div(cy, M), ieee_div(cz, M), M);
     if (quad) {
         float Q[6];
@@ -500,8 +519,13 @@ __device__ __forceinline__ void oct_quad_inner(int p, const OctRec &r, const Oct
 __device__ __forceinline__ void oct_summ_inner(int p, const OctRec &r, OctRec *nodes, float4 *quad) {
     const int c0 = r.topo.z, nch = oct_nchild(r);
     float M = 0.0f, cx = 0.0f, cy = 0.0f, cz = 0.0f;
-    for (int k = 0; k < nch; ++k) {
-        const float4 c = nodes[c0 + k].com;
+    float4 ch[8];  // all loads in flight (past the last child: the last again)
+#pragma unroll
+    for (int k = 0; k < 8; ++k) ch[k] = nodes[c0 + (k < nch ? k : nch - 1)].com;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        if (k >= nch) continue;
+        const float4 c = ch[k];
         M += c.w;
         cx = cx + c.x * c.w;
         cy = cy + c.y * c.w;
@@ -516,44 +540,42 @@ __device__ __forceinline__ void oct_summ_inner(int p, const OctRec &r, OctRec *n
     if (quad) oct_quad_inner(p, r, nodes, quad, com);
 }
 
-__global__ __launch_bounds__(kSummThreads) void k_oct_summ_local(const float4 *__restrict__ bodies, int64_t n,
+__global__ __launch_bounds__(kOctSummBodies) void k_oct_summ_local(const float4 *__restrict__ bodies, int64_t n,
                                                         OctRec *nodes, const int32_t *__restrict__ leaf_start,
                                                         const uint32_t *__restrict__ misc, uint32_t *flags,
                                                         uint32_t *glist, int64_t glist_cap, float4 *quad,
                                                         uint32_t *err) {
-    const int64_t lo = (int64_t)blockIdx.x * kSummBodies, hi = lo + kSummBodies;
-    const int64_t end = hi < n ? hi : n;
-    const int64_t T = misc[0];
-    for (int64_t i = lo + threadIdx.x; i < end; i += blockDim.x) {
-        const int s = leaf_start[i];
-        if (s < 0) continue;
-        if (s >= T) { atomicOr(err, 4u); continue; }
-        const int4 t = nodes[s].topo;
-        if (t.x != (int)i || t.y < 1 || (int64_t)t.x + t.y > n || t.z >= 0) { atomicOr(err, 4u); continue; }
-        oct_summ_leaf(s, t, bodies, nodes, quad);
-        int parent = t.w;
-        for (int hops = 0; parent >= 0; ++hops) {
-            // parents sit in lower slots than their children; a valid tree
-            // is at most kOctLevels deep
-            if (parent >= s || hops > kOctLevels) { atomicOr(err, 4u); break; }
-            const OctRec r = nodes[parent];
-            const int4 tp = r.topo;
-            const bool local = tp.x >= lo && (int64_t)tp.x + tp.y <= hi;
-            if (!local) {
-                const uint32_t k = atomicAdd(&glist[0], 1u);
-                if (k < glist_cap) glist[64 + k] = (uint32_t)parent;
-                else atomicOr(err, 4u);
-                break;
-            }
-            if (arrive(&flags[parent]) + 1u < (uint32_t)oct_nchild(r)) break;
-            if (tp.z <= parent || tp.z + oct_nchild(r) > T || tp.w >= parent) { atomicOr(err, 4u); break; }
-            oct_summ_inner(parent, r, nodes, quad);
-            parent = tp.w;
+    const int64_t lo = (int64_t)blockIdx.x * kOctSummBodies, hi = lo + kOctSummBodies;
+    const int64_t T = misc[0], i = lo + threadIdx.x;
+    if (i >= n) return;
+    const int s = leaf_start[i];
+    if (s < 0) return;
+    if (s >= T) { atomicOr(err, 4u); return; }
+    const int4 t = nodes[s].topo;
+    if (t.x != (int)i || t.y < 1 || (int64_t)t.x + t.y > n || t.z >= 0) { atomicOr(err, 4u); return; }
+    oct_summ_leaf(s, t, bodies, nodes, quad);
+    int parent = t.w;
+    for (int hops = 0; parent >= 0; ++hops) {
+        // parents sit in lower slots than their children; a valid tree
+        // is at most kOctLevels deep
+        if (parent >= s || hops > kOctLevels) { atomicOr(err, 4u); break; }
+        const OctRec r = nodes[parent];
+        const int4 tp = r.topo;
+        const bool local = tp.x >= lo && (int64_t)tp.x + tp.y <= hi;
+        if (!local) {
+            const uint32_t k = atomicAdd(&glist[0], 1u);
+            if (k < glist_cap) glist[64 + k] = (uint32_t)parent;
+            else atomicOr(err, 4u);
+            break;
         }
+        if (arrive(&flags[parent]) + 1u < (uint32_t)oct_nchild(r)) break;
+        if (tp.z <= parent || tp.z + oct_nchild(r) > T || tp.w >= parent) { atomicOr(err, 4u); break; }
+        oct_summ_inner(parent, r, nodes, quad);
+        parent = tp.w;
     }
 }
 
-// Middle pass (as the linear BVH's): workgroup g owns kSummMidBodies bodies
+// Middle pass (as the linear BVH's): workgroup g owns kOctSummMid bodies
 // and the queued parents whose first body lies there, climbs while the node
 // stays inside, and forwards a parent that leaves the range in place of the
 // arrival.
@@ -561,7 +583,7 @@ __global__ __launch_bounds__(1024) void k_oct_summ_mid(OctRec *nodes, const uint
                                                        uint32_t *flags, const uint32_t *gin, uint32_t *gout,
                                                        int64_t qcap, float4 *quad, uint32_t *err) {
     const int64_t T = misc[0];
-    const int64_t lo = (int64_t)blockIdx.x * kSummMidBodies, hi = lo + kSummMidBodies;
+    const int64_t lo = (int64_t)blockIdx.x * kOctSummMid, hi = lo + kOctSummMid;
     const uint32_t cnt = gin[0] < qcap ? gin[0] : (uint32_t)qcap;
     for (uint32_t j = threadIdx.x; j < cnt; j += blockDim.x) {
         int parent = (int)gin[64 + j];
@@ -620,63 +642,40 @@ inline OctKeys make_keys(const uint64_t *keys, const OctBuffers &ob, int64_t n, 
 
 }  // namespace
 
-void launch_octree_keys(const float *x, const float *y, const float *z, int64_t n, const float *bbox6,
-                        int max_depth, OctBuffers &ob, uint64_t *keys, uint32_t *idx, uint32_t *idx_alt,
-                        hipStream_t s) {
+void launch_octree_keys(const float *x, const float *y, const float *z, int64_t n, const float *partials, int blocks,
+                        float *bbox6, int max_depth, float theta, const SortPlan &plan, OctBuffers &ob, uint64_t *keys,
+                        uint32_t *idx, uint64_t *keys_alt, uint32_t *idx_alt, uint32_t *status, hipStream_t s) {
     if (n <= 0) return;
     const int levels = max_depth + 2;
-    const unsigned g = blocks_for(n, 256);
-    // With lower-level digits the low word is sorted first from `keys`/`idx`;
-    // otherwise the high word is sorted directly from `keys`/`idx_alt`.
+    int64_t g = (n + 255) / 256;
+    if (g > 256) g = 256;  // every workgroup adds its digit counts to the histograms
+    uint64_t *k = plan.from_alt ? keys_alt : keys;
+    uint32_t *v = plan.from_alt ? idx_alt : idx;
     if (levels > kOctHiLevels)
-        hipLaunchKernelGGL(k_oct_keys<true>, dim3(g), dim3(256), 0, s, x, y, z, n, bbox6, levels, ob.key_hi, keys,
-                           ob.key_lo, idx);
+        hipLaunchKernelGGL(k_oct_keys<true>, dim3((unsigned)g), dim3(256), 0, s, x, y, z, n, partials, blocks, bbox6,
+                           levels, theta, ob.thr, k, ob.key_lo, v, status, plan.passes, plan.shift);
     else
-        hipLaunchKernelGGL(k_oct_keys<false>, dim3(g), dim3(256), 0, s, x, y, z, n, bbox6, levels, keys,
-                           (uint64_t *)nullptr, (uint64_t *)nullptr, idx_alt);
+        hipLaunchKernelGGL(k_oct_keys<false>, dim3((unsigned)g), dim3(256), 0, s, x, y, z, n, partials, blocks, bbox6,
+                           levels, theta, ob.thr, k, (uint64_t *)nullptr, v, status, plan.passes, plan.shift);
 }
 
-void launch_octree_sort(int64_t n, int max_depth, OctBuffers &ob, uint64_t *keys, uint32_t *idx,
-                        uint64_t *keys_alt, uint32_t *idx_alt, uint32_t *sort_status, uint32_t *err,
-                        hipStream_t s) {
+void launch_octree_topology(int64_t n, const float *bbox6, int leaf_size, int max_depth, OctBuffers &ob,
+                            const uint64_t *keys, const uint32_t *idx_in, uint32_t *idx, int32_t *leaf_start,
+                            uint32_t *err, hipStream_t s) {
     if (n <= 0) return;
-    const int levels = max_depth + 2;
-    const unsigned g = blocks_for(n, 256);
-    if (levels > kOctHiLevels) {
-        const int lo_bits = 3 * (levels - kOctHiLevels);
-        // low word: (keys, idx) -> (keys_alt, idx_alt) after an odd pass count
-        int passes = (lo_bits + 7) / 8;
-        if (!(passes & 1)) ++passes;
-        launch_radix_sort_u64(keys, idx, keys_alt, idx_alt, n, passes, sort_status, err, s);
-        if (n == 1) launch_fill_u32(idx_alt, 0u, 1, s);
-        hipLaunchKernelGGL(k_gather_u64, dim3(g), dim3(256), 0, s, ob.key_hi, idx_alt, n, keys);
-    }
-    // high word (63 bits, 8 passes): (keys, idx_alt) -> (keys, idx_alt)
-    launch_radix_sort_u64(keys, idx_alt, keys_alt, idx, n, 8, sort_status, err, s);
-    if (levels > kOctHiLevels)
-        hipLaunchKernelGGL(k_gather_u64, dim3(g), dim3(256), 0, s, ob.key_lo, idx_alt, n, ob.lo_sorted);
-}
-
-void launch_octree_topology(int64_t n, const float *bbox6, int leaf_size, int max_depth, float theta,
-                            OctBuffers &ob, const uint64_t *keys, const uint32_t *idx_alt, uint32_t *idx,
-                            int32_t *leaf_start, uint32_t *err, hipStream_t s) {
-    if (n <= 0) return;
-    const int levels = max_depth + 2;
     const OctKeys K = make_keys(keys, ob, n, max_depth);
     const unsigned g = blocks_for(n, 256), gc = blocks_for(ob.cap, 256);
-    hipLaunchKernelGGL(k_oct_count, dim3(g), dim3(256), 0, s, K, leaf_size, ob.nown);
-    launch_scan_u32(ob.nown, ob.nbase, n, ob.scan_ws, ob.misc, s);
-    launch_fill_u32(ob.occ, 0u, ob.cap, s);
+    hipLaunchKernelGGL(k_oct_count, dim3(g), dim3(256), 0, s, K, leaf_size, ob.nown,
+                       scan_fused(n) ? ob.sums_own() : nullptr);
+    launch_scan_u32(ob.nown, ob.nbase, n, ob.sums_own(), ob.misc, s);
     hipLaunchKernelGGL(k_oct_nodes, dim3(g), dim3(256), 0, s, K, leaf_size, ob.nbase, ob.cap, ob.nfirst, ob.ncount,
                        ob.nparent, ob.nmeta, ob.occ, err);
-    hipLaunchKernelGGL(k_oct_nchild, dim3(gc), dim3(256), 0, s, ob.misc, ob.cap, ob.nmeta, ob.occ, ob.cb);
-    launch_scan_u32(ob.cb, ob.cb, ob.cap, ob.scan_ws, ob.misc + 1, s);
-    hipLaunchKernelGGL(k_oct_levels, dim3(1), dim3(64), 0, s, bbox6, levels, theta, ob.thr);
-    launch_fill_u32((uint32_t *)leaf_start, 0xFFFFFFFFu, n, s);
+    hipLaunchKernelGGL(k_oct_nchild, dim3(gc), dim3(256), 0, s, ob.misc, ob.cap, ob.nmeta, ob.occ, ob.cb,
+                       scan_fused(ob.cap) ? ob.sums_child() : nullptr);
+    launch_scan_u32(ob.cb, ob.cb, ob.cap, ob.sums_child(), ob.misc + 1, s, ob.misc);
     hipLaunchKernelGGL(k_oct_emit, dim3(gc), dim3(256), 0, s, ob.misc, ob.cap, 1, bbox6, K, ob.thr, ob.nfirst,
                        ob.ncount, ob.nparent, ob.nmeta, ob.occ, ob.cb, ob.nodes, ob.centre, leaf_start, err);
-    hipLaunchKernelGGL(k_oct_leafsort, dim3(g), dim3(256), 0, s, n, leaf_start, ob.nodes, ob.cap, idx_alt, idx,
-                       err);
+    hipLaunchKernelGGL(k_oct_leafsort, dim3(g), dim3(256), 0, s, n, leaf_start, ob.nodes, ob.cap, idx_in, idx, err);
 }
 
 void launch_octree_forest_build(const float *x, const float *y, const float *z, int64_t n, int nsys,
@@ -727,15 +726,15 @@ void launch_octree_forest_topology(int64_t n, int nsys, const float *bbox6, cons
     K.lv_tab = lv_tab;
     K.leaf_tab = leaf_tab;
     const unsigned g = blocks_for(n, 256), gc = blocks_for(ob.cap, 256);
-    hipLaunchKernelGGL(k_oct_count, dim3(g), dim3(256), 0, s, K, 0, ob.nown);
-    launch_scan_u32(ob.nown, ob.nbase, n, ob.scan_ws, ob.misc, s);
-    launch_fill_u32(ob.occ, 0u, ob.cap, s);
+    hipLaunchKernelGGL(k_oct_count, dim3(g), dim3(256), 0, s, K, 0, ob.nown,
+                       scan_fused(n) ? ob.sums_own() : nullptr);
+    launch_scan_u32(ob.nown, ob.nbase, n, ob.sums_own(), ob.misc, s);
     hipLaunchKernelGGL(k_oct_nodes, dim3(g), dim3(256), 0, s, K, 0, ob.nbase, ob.cap, ob.nfirst, ob.ncount,
                        ob.nparent, ob.nmeta, ob.occ, err);
-    hipLaunchKernelGGL(k_oct_nchild, dim3(gc), dim3(256), 0, s, ob.misc, ob.cap, ob.nmeta, ob.occ, ob.cb);
-    launch_scan_u32(ob.cb, ob.cb, ob.cap, ob.scan_ws, ob.misc + 1, s);
+    hipLaunchKernelGGL(k_oct_nchild, dim3(gc), dim3(256), 0, s, ob.misc, ob.cap, ob.nmeta, ob.occ, ob.cb,
+                       scan_fused(ob.cap) ? ob.sums_child() : nullptr);
+    launch_scan_u32(ob.cb, ob.cb, ob.cap, ob.sums_child(), ob.misc + 1, s, ob.misc);
     hipLaunchKernelGGL(k_oct_levels_forest, dim3((unsigned)nsys), dim3(64), 0, s, bbox6, lv_tab, sys_prm, ob.thr);
-    launch_fill_u32((uint32_t *)leaf_start, 0xFFFFFFFFu, n, s);
     hipLaunchKernelGGL(k_oct_emit, dim3(gc), dim3(256), 0, s, ob.misc, ob.cap, nsys, bbox6, K, ob.thr, ob.nfirst,
                        ob.ncount, ob.nparent, ob.nmeta, ob.occ, ob.cb, ob.nodes, ob.centre, leaf_start, err);
     hipLaunchKernelGGL(k_oct_leafsort, dim3(g), dim3(256), 0, s, n, leaf_start, ob.nodes, ob.cap, idx_alt, idx,
@@ -747,13 +746,10 @@ void launch_octree_summaries(const float4 *bodies, int64_t n, OctBuffers &ob, co
     if (n <= 0) return;
     // queue layout: local -> middle at glist, middle -> global at glist + cap + 64
     uint32_t *gmid = ob.glist + ob.cap + 64;
-    launch_fill_u32(ob.flags, 0u, ob.cap, s);
-    launch_fill_u32(ob.glist, 0u, 64, s);
-    launch_fill_u32(gmid, 0u, 64, s);
-    hipLaunchKernelGGL(k_oct_summ_local, dim3(blocks_for(n, kSummBodies)), dim3(kSummThreads), 0, s, bodies, n, ob.nodes,
+    hipLaunchKernelGGL(k_oct_summ_local, dim3(blocks_for(n, kOctSummBodies)), dim3(kOctSummBodies), 0, s, bodies, n, ob.nodes,
                        leaf_start, ob.misc, ob.flags, ob.glist, ob.cap, quad, err);
-    const unsigned mblocks = blocks_for(n, kSummMidBodies);
-    const bool mid = mblocks >= kSummMidMinBlocks;  // see launch_lbvh_summaries
+    const unsigned mblocks = blocks_for(n, kOctSummMid);
+    const bool mid = mblocks >= kOctSummMidMinBlocks;
     if (mid)
         hipLaunchKernelGGL(k_oct_summ_mid, dim3(mblocks), dim3(1024), 0, s, ob.nodes, ob.misc, ob.flags, ob.glist, gmid,
                            ob.cap, quad, err);
