@@ -197,13 +197,14 @@ int nbg_sys_walk_stats(nbg_sys *sys, uint64_t *out4);
 
 /* Waves that share a group of targets in the tree walks (no reference
  * counterpart: a schedule choice).  0 (the default) chooses by size: small
- * systems fill the GPU with up to 4 waves per 16 targets (FAST) or, up to
- * 65,536 bodies, 16 waves per 64 targets (ORDERED), within 4,096 waves in
- * all; larger ones use 1.  Results are the same bits for every choice: FAST
- * sums each target's interactions in four fixed classes, which the waves
- * share out; ORDERED computes each frontier subtree's result from zero, as
- * the reference's recursion does, and adds it where the walk meets it.  A
- * split ORDERED walk keeps 1,536 bytes per body of results in HBM. */
+ * systems fill the GPU with up to 4 waves per 16 targets (FAST) or 8 or 16
+ * (ORDERED); larger ones use 1.  Other values are taken as the nearest that
+ * the walk offers.  Results are the same bits for every choice: FAST sums
+ * each target's interactions in four fixed classes, which the waves share
+ * out; ORDERED computes each opened node's result from its children's alone,
+ * as the reference's recursion does.  By default a linear BVH of 16,385 to
+ * 65,536 bodies is walked with up to 16 waves per 64 targets, which keep
+ * 1,536 bytes per body of results in HBM. */
 int nbg_sys_set_walk_split(nbg_sys *sys, int32_t waves);
 
 /* Per-phase device time (ms) of the last force pass, measured with HIP events

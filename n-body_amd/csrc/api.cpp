@@ -86,11 +86,10 @@ struct nbg_sys {
     int64_t fmm_item_cap = 0, fmm_pool_cap = 0;
     int fmm_seed_cap = 0;
     int fmm_shift = 0;  // capacity doublings after passes that outgrew the pool
-    // split ORDERED walks of small systems: per-target results of the frontier
-    // subtrees (see WalkArgs::split); split_req 0 = automatic
+    int split_req = 0;  // waves that share a group of targets; 0 = automatic
+    // ORDERED split of a linear BVH: the frontier subtrees' results
     float *split_part = nullptr;
     int64_t split_cap = 0;
-    int split_req = 0;
     // passive-point walks (nbg_sys_accelerations_at): one buffer that grows
     // to the largest target count seen and is kept for later calls
     void *pts = nullptr;
@@ -219,14 +218,22 @@ int ensure_fmm(nbg_sys *s) {
     return NBG_OK;
 }
 
-// Waves per group of targets in the system's tree walk (1 for the other
-// solvers): chosen by size, or as requested (FAST walks use at most 4).
-int split_of(const nbg_sys *s) {
-    if (s->prm.solver == NBG_NAIVE || s->prm.solver == NBG_IMPLICIT_FMM) return 1;
-    if (s->prm.sum_mode == NBG_SUM_FAST)
-        return s->split_req > 0 ? std::min(s->split_req, 4) : fast_split_waves((s->n + 63) / 64);
-    if (s->n > kOrderedSplitMaxBodies) return 1;
-    return s->split_req > 0 ? s->split_req : ordered_split_waves(s->n);
+// Waves that share a group of targets in a walk of nt of them (1 for the
+// solvers without a tree walk): chosen by size, or as requested.
+int split_of(const nbg_sys *s, int64_t nt) {
+    const int32_t solver = s->prm.solver;
+    if (solver == NBG_NAIVE || solver == NBG_IMPLICIT_FMM) return 1;
+    if (s->split_req > 0) return s->split_req;
+    const int64_t groups = (nt + 63) / 64;
+    const bool octree = solver == NBG_BARNES_HUT || solver == NBG_BARNES_HUT_QUADRUPOLE;
+    return s->prm.sum_mode == NBG_SUM_FAST ? fast_split_waves(groups) : ordered_split_waves(groups, octree);
+}
+
+// Waves per 64 targets of the system's own walk when it is split by subtrees.
+int subtree_split_of(const nbg_sys *s) {
+    if (s->prm.sum_mode != NBG_SUM_ORDERED || s->split_req > 0) return 1;
+    if (s->prm.solver != NBG_LINEAR_BVH && s->prm.solver != NBG_LINEAR_BVH_QUADRUPOLE) return 1;
+    return ordered_subtree_waves(s->n);
 }
 
 void free_split(nbg_sys *s) {
@@ -238,7 +245,7 @@ void free_split(nbg_sys *s) {
 // Allocates the ORDERED split walk's results when the system's walk splits
 // (no-op otherwise or when the current ones are large enough).
 int ensure_split(nbg_sys *s) {
-    if (s->prm.sum_mode == NBG_SUM_FAST || split_of(s) <= 1 || s->split_cap >= s->n) return NBG_OK;
+    if (subtree_split_of(s) <= 1 || s->split_cap >= s->n) return NBG_OK;
     if (s->stream) NBG_HIP(hipStreamSynchronize(s->stream));
     free_split(s);
     const int64_t n = s->n > 0 ? s->n : 1;
@@ -411,15 +418,7 @@ int enqueue_force_pass(nbg_sys *s) {
         fa.err = s->err_word();
         launch_fmm(fa, st);
     } else {
-        WalkArgs wa = walk_args(s);
-        const int k = split_of(s);
-        if (p.sum_mode == NBG_SUM_FAST) {
-            wa.split = k;
-        } else if (k > 1 && s->split_part && s->split_cap >= s->n) {
-            wa.split = k;
-            wa.split_part_f = s->split_part;
-            wa.split_stride = s->n;
-        }
+        const WalkArgs wa = walk_args(s);
         const int stats = s->walk_stats ? 2 : (s->counting ? 1 : 0);
         launch_walk(s, wa, stats);
     }
@@ -455,6 +454,12 @@ WalkArgs walk_args(nbg_sys *s) {
     wa.counts = s->counts();
     wa.err = s->err_word();
     wa.quad = is_quad(p.solver) ? s->quad : nullptr;
+    wa.split = split_of(s, n);
+    if (const int k = subtree_split_of(s); k > 1 && s->split_part && s->split_cap >= n) {
+        wa.split = k;
+        wa.split_part_f = s->split_part;
+        wa.split_stride = n;
+    }
     return wa;
 }
 
@@ -635,7 +640,8 @@ int walk_points(nbg_sys *s, int64_t nt, const float *tx, const float *ty, const 
     launch_gather(pb.t3, pb.t3 + nt, pb.t3 + 2 * nt, pb.t3, pb.i2, nt, pb.t4, st);
     WalkArgs wa = walk_args(s);
     wa.nt = nt;
-    if (s->prm.sum_mode == NBG_SUM_FAST) wa.split = fast_split_waves((nt + 63) / 64);
+    wa.split = split_of(s, nt);
+    wa.split_part_f = nullptr;
     wa.targets = pb.t4;
     wa.perm = pb.i2;
     wa.ax = pb.a3;

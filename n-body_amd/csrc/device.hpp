@@ -29,40 +29,45 @@ __device__ __forceinline__ float ieee_div(float a, float b) { return a / b; }
 // Newton steps (within ~2^-52 of 1/d).  The exact quotient of two binary32
 // numbers is either a binary32 number or at least ~2^-49 (relative) away
 // from every binary32 rounding midpoint (it can never lie on one), so an FP64
-// value within ~2^-51 of it rounds to the IEEE quotient.  d = 0, inf or NaN
-// take the IEEE division itself.  The identity is checked on 10^8 random
-// pairs with the reciprocal perturbed by up to 2 FP64 ulp (CPU test).
-__device__ __forceinline__ void ieee_div3(float nx, float ny, float nz, float d, float &qx, float &qy, float &qz) {
-    if (__builtin_expect(d > 0.0f && d < __builtin_huge_valf(), 1)) {
-        const double dd = (double)d;
-        double r = __builtin_amdgcn_rcp(dd);
-        r = __builtin_fma(r, __builtin_fma(-dd, r, 1.0), r);
-        r = __builtin_fma(r, __builtin_fma(-dd, r, 1.0), r);
-        qx = (float)((double)nx * r);
-        qy = (float)((double)ny * r);
-        qz = (float)((double)nz * r);
-    } else {
-        qx = ieee_div(nx, d);
-        qy = ieee_div(ny, d);
-        qz = ieee_div(nz, d);
-    }
+// value within ~2^-51 of it rounds to the IEEE quotient.  The identity is
+// checked on 10^8 random pairs with the reciprocal perturbed by up to 2 FP64
+// ulp (CPU test).  Not for d = 0, inf or NaN.
+__device__ __forceinline__ void quotients3(float nx, float ny, float nz, float d, float &qx, float &qy, float &qz) {
+    const double dd = (double)d;
+    double r = __builtin_amdgcn_rcp(dd);
+    r = __builtin_fma(r, __builtin_fma(-dd, r, 1.0), r);
+    r = __builtin_fma(r, __builtin_fma(-dd, r, 1.0), r);
+    qx = (float)((double)nx * r);
+    qy = (float)((double)ny * r);
+    qz = (float)((double)nz * r);
 }
 
 // Gravity::particleParticle (Physics/Rules/Gravity.h:199-209) with the
 // reference's FP32 operation order: R = p - a, r = sqrt(R.R + eps2),
-// -R m G / (r (r r)); zero when the positions are equal.  Compile without
-// FMA contraction.
+// -R m G / (r (r r)); zero when the positions are equal.  Denominators of 0,
+// inf or NaN take the IEEE division itself, on a branch that a wave enters
+// only if one of its lanes needs it: the common path has no branches, so
+// that several calls overlap.  Compile without FMA contraction.
 __device__ __forceinline__ void pp_exact(float bx, float by, float bz, float bm, float px, float py, float pz,
                                          float G, float eps2, float &vx, float &vy, float &vz) {
-    if (bx == px && by == py && bz == pz) {
-        vx = 0.0f; vy = 0.0f; vz = 0.0f;
-        return;
-    }
+    const bool same = bx == px && by == py && bz == pz;
     const float Rx = px - bx, Ry = py - by, Rz = pz - bz;
     const float r2 = Rx * Rx + Ry * Ry + Rz * Rz;
     const float r = ieee_sqrt(r2 + eps2);
     const float r3 = r * (r * r);
-    ieee_div3((-Rx * bm) * G, (-Ry * bm) * G, (-Rz * bm) * G, r3, vx, vy, vz);
+    const float nx = (-Rx * bm) * G, ny = (-Ry * bm) * G, nz = (-Rz * bm) * G;
+    quotients3(nx, ny, nz, r3, vx, vy, vz);
+    const bool odd = !same && !(r3 > 0.0f && r3 < __builtin_huge_valf());
+    if (__builtin_expect(__ballot(odd) != 0, 0)) {
+        if (odd) {
+            vx = ieee_div(nx, r3);
+            vy = ieee_div(ny, r3);
+            vz = ieee_div(nz, r3);
+        }
+    }
+    vx = same ? 0.0f : vx;
+    vy = same ? 0.0f : vy;
+    vz = same ? 0.0f : vz;
 }
 
 // ---------------------------------------------------------------- quadrupole

@@ -174,11 +174,12 @@ int walk_tpl(const nbg_batch *b) {
     return lbvh && b->sum_mode == NBG_SUM_FAST ? b->tpl : 1;
 }
 
-// Waves per 16 targets of the forest's FAST walk: as requested, or by the
-// number of groups, as for one system (the bits do not depend on it).
+// Waves that share a group of the forest's targets: as requested (FAST
+// walks), or by the number of groups, as for one system (the bits do not
+// depend on it).
 int forest_split(const nbg_batch *b) {
-    if (b->sum_mode != NBG_SUM_FAST) return 1;
-    return b->split_req > 0 ? std::min(b->split_req, 4) : fast_split_waves(b->nwaves);
+    if (b->sum_mode != NBG_SUM_FAST) return ordered_split_waves(b->nwaves, is_octree_solver(b->solver));
+    return b->split_req > 0 ? b->split_req : fast_split_waves(b->nwaves);
 }
 
 int ensure_quad(nbg_batch *b, int64_t slots) {

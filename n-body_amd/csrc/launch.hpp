@@ -355,27 +355,38 @@ struct WalkArgs {
     // Quadrupole trees: second moments per node slot (2 float4, layout in
     // device.hpp); null for monopole trees.
     const float4 *quad = nullptr;
-    // Small systems: waves that share a group of targets (1 = none).  FAST: 1,
-    // 2 or 4 waves per 16 targets.  ORDERED: waves per 64 targets, each storing
-    // its frontier subtrees' results in split_part_f (kOrderedSplitSlots x 3
-    // floats per target, split_stride floats apart) for a second kernel.
+    // Waves that share 16 targets.  FAST: 1, 2 or 4.  ORDERED: 8 or 16 by
+    // frames (2 and 4 read as 8), 1: the recursion, 64 targets a wave.
+    // ORDERED with split_part_f: that many waves per 64 targets, which leave
+    // their frontier subtrees' results there (kOrderedSplitSlots x 3 floats
+    // per target, split_stride floats apart) for a second kernel.
     int split = 1;
     float *split_part_f = nullptr;
     int64_t split_stride = 0;
 };
 
-// ORDERED split: one result per frontier subtree (at most kOrderedSplitSlots)
-// per target, for systems of at most kOrderedSplitMaxBodies bodies.
+// ORDERED waves per 16 targets for a walk by frames of `groups` groups of 64
+// targets, 1: none.  Measured, walk us at n bodies, theta 0.5, leaf 16:
+// octree, 8 / 16 waves / recursion (the split that was here before): 1,000 59
+// / 49 / 315; 3,000 94 / 102; 10,000 235 / 294 / 1,045; 200,000 3,777 / 5,685
+// / 5,393; 400,000 8,911 / - / 7,426.  Linear BVH, 8 / 16 / split: 3,000 142 /
+// 118 / 478; 5,000 272 / 267 / 720; 10,000 891 / 987 / 1,026; 16,000 1,457 /
+// 2,407 / 1,595: its frames outgrow the slots.
+inline int ordered_split_waves(int64_t groups, bool octree) {
+    if (octree) return groups <= 32 ? 16 : groups <= 4096 ? 8 : 1;
+    return groups <= 80 ? 16 : groups <= 256 ? 8 : 1;
+}
+
+// ORDERED split of one linear BVH of n bodies past that: waves per 64 targets
+// within 4,096 waves (1: the chip is full without), one result per frontier
+// subtree.
 constexpr int kOrderedSplitSlots = 128;
 constexpr int64_t kOrderedSplitMaxBodies = 65536;
-// ORDERED split waves per group for a system of n bodies (1: the chip is
-// full): the most waves, up to 16 per group, that keep the launch within
-// 4,096 waves (16 per CU; measured: wider launches of the split walks run
-// slower from 30k bodies up).
-inline int ordered_split_waves(int64_t n) {
-    if (n > kOrderedSplitMaxBodies || n < 1) return 1;
+inline int ordered_subtree_waves(int64_t n) {
+    const int64_t groups = (n + 63) / 64;
+    if (ordered_split_waves(groups, false) > 1 || n > kOrderedSplitMaxBodies) return 1;
     int k = 1;
-    while (k < 16 && (n + 63) / 64 * k * 2 <= 4096) k *= 2;
+    while (k < 16 && groups * 2 * k <= 4096) k *= 2;
     return k;
 }
 // FAST waves per 16 targets for a walk of `groups` groups of 64 targets: the

@@ -1,0 +1,46 @@
+"""The ORDERED walks by frames (16 targets per workgroup, the opened nodes
+listed level by level and evaluated from the last one up) give the oracle's
+bits and counts where they can go wrong: groups of 1, 15, 16, 17 and 63
+targets, a root that is a leaf, leaves of one body and of more bodies than a
+row step or a whole listing holds, coincident bodies without softening (whose
+terms are zero), more opened nodes than a workgroup's slots (the recursion
+takes over) and points walked from outside the tree."""
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _same_bits(a, b):
+    """Equal bits, or both NaN (a NaN's sign is not defined by 0/0)."""
+    return np.all((a.view(np.uint32) == b.view(np.uint32)) | (np.isnan(a) & np.isnan(b)))
+
+# n, theta, leaf, eps2, coincident bodies
+CASES = [(1, 0.5, 16, 1e-4, 0), (15, 0.5, 1, 1e-4, 0), (16, 0.5, 16, 0.0, 4), (17, 0.3, 2, 0.0, 6),
+         (63, 0.8, 5, 1e-4, 0), (257, 0.5, 4, 0.0, 12), (1000, 0.3, 64, 1e-5, 0), (1500, 0.7, 200, 1e-4, 0),
+         (3000, 0.05, 2, 1e-4, 0), (5121, 0.5, 8, 1e-4, 9), (16385, 0.9, 16, 1e-4, 0)]
+
+
+@pytest.mark.parametrize("solver", ["LINEAR_BVH", "BARNES_HUT", "LINEAR_BVH_QUADRUPOLE", "BARNES_HUT_QUADRUPOLE"])
+@pytest.mark.parametrize("n,theta,leaf,eps2,same", CASES)
+def test_frames_bitexact(nbg, orc, gpu_ctx, n, theta, leaf, eps2, same, solver):
+    print(f"[frames] {solver} n={n} theta={theta} leaf={leaf}", flush=True)
+    b = nbg.plummer(n, seed=7000 + n)
+    for k in range(same):
+        j, i = n - 1 - k, k // 2
+        b.x[j], b.y[j], b.z[j] = b.x[i], b.y[i], b.z[i]
+    p = nbg.default_params()
+    p.solver, p.theta, p.leaf_size, p.morton_bits, p.eps2 = getattr(nbg, solver), theta, leaf, 63, eps2
+    p.sum_mode = nbg.SUM_ORDERED
+    kind = {"LINEAR_BVH": 1, "BARNES_HUT": 0, "LINEAR_BVH_QUADRUPOLE": 4, "BARNES_HUT_QUADRUPOLE": 3}[solver]
+    t = orc.Tree(kind, b.x, b.y, b.z, b.m, theta=theta, leaf=leaf, bits=63, eps2=eps2)
+    want, pp, npc = t.accel(b.x, b.y, b.z, counts=True)
+    s = nbg.System(gpu_ctx, p, n)
+    s.set_state(b)
+    for k in (8, 16, 0):
+        s.set_walk_split(k)
+        acc = s.update_accelerations()
+        assert _same_bits(acc, want), f"waves {k}"
+        assert s.counts() == (int(pp.sum()), int(npc.sum())), f"waves {k}"
+    s.close()
