@@ -218,6 +218,11 @@ int ensure_fmm(nbg_sys *s) {
     return NBG_OK;
 }
 
+// Whether the system's walk takes its targets in compact groups (targets.hip).
+bool grouped(const nbg_sys *s) {
+    return s->n >= kGroupMin && s->prm.solver != NBG_NAIVE && s->prm.solver != NBG_IMPLICIT_FMM;
+}
+
 // Waves that share a group of targets in a walk of nt of them (1 for the
 // solvers without a tree walk): chosen by size, or as requested.
 int split_of(const nbg_sys *s, int64_t nt) {
@@ -384,6 +389,8 @@ int enqueue_force_pass(nbg_sys *s) {
         launch_lbvh_summaries(s->bodies, n, s->nodes, s->leaf_start, 2 * n, s->flags, s->glist, s->bmin, s->bmax,
                               p.theta, s->err_word(), st, nullptr, nullptr, 0, quad);
     }
+    // the summaries' queues and the sort's other half are free by now
+    if (grouped(s)) launch_group_targets(s->bodies, s->idx, n, (float4 *)s->glist, (uint32_t *)s->keys_alt, st);
     mark(s, 6);
     if (p.solver == NBG_IMPLICIT_FMM) {
         FmmArgs fa;
@@ -437,8 +444,8 @@ WalkArgs walk_args(nbg_sys *s) {
     wa.n = n;
     wa.bodies = s->bodies;
     wa.nt = n;
-    wa.targets = s->bodies;
-    wa.perm = s->idx;
+    wa.targets = grouped(s) ? (const float4 *)s->glist : s->bodies;
+    wa.perm = grouped(s) ? (const uint32_t *)s->keys_alt : s->idx;
     wa.nodes = s->nodes;
     wa.onodes = s->ob.nodes;
     wa.levels = p.max_depth + 2;

@@ -94,6 +94,7 @@ struct nbg_batch {
     // targets per lane asked for (the autotuner's bodies-per-wavefront
     // choice): a hint that the present walks do not need
     int32_t tpl = 1;
+    bool grouped = false;   // a member takes its targets in groups (kGroupMin)
     int32_t split_req = 0;  // waves per group of the FAST walk: 0 = by size
     float *x() { return st[0]; }
     float *y() { return st[1]; }
@@ -130,7 +131,7 @@ bool is_octree_solver(int32_t solver) { return solver == NBG_BARNES_HUT || solve
 
 void free_octree(OctBuffers &o) {
     void *ptrs[] = {o.key_hi, o.key_lo, o.lo_sorted, o.nown, o.nbase, o.nfirst, o.ncount, o.nparent, o.nmeta,
-                    o.occ, o.cb, o.flags, o.glist, o.scan_ws, o.nodes, o.centre, o.thr, o.misc};
+                    o.occ, o.cb, o.flags, o.glist, o.targets, o.scan_ws, o.nodes, o.centre, o.thr, o.misc};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     o = OctBuffers{};
@@ -225,6 +226,7 @@ int ensure_octree(nbg_batch *b) {
             if (r == NBG_OK) r = dalloc(ptr, count);
         };
         A(&o.key_hi, n); A(&o.key_lo, n); A(&o.lo_sorted, n); A(&o.nown, n); A(&o.nbase, n);
+        A(&o.targets, n);
         A(&o.nfirst, cap); A(&o.ncount, cap); A(&o.nparent, cap); A(&o.nmeta, cap);
         A(&o.occ, cap); A(&o.cb, cap); A(&o.flags, cap); A(&o.glist, 2 * (cap + 64));
         A(&o.scan_ws, oct_scan_words(n, cap));
@@ -252,6 +254,7 @@ int upload_tables(nbg_batch *b) {
     std::vector<MacParam> mp(S);
     int64_t off = 0, w = 0;
     b->all_soft = true;
+    b->grouped = false;
     b->max_levels = 0;
     if (S) b->solver = b->sys[0].p.solver;
     const int64_t width = 64;  // targets per group
@@ -269,6 +272,7 @@ int upload_tables(nbg_batch *b) {
         prm[i] = make_float4(m.p.G, m.p.eps2, m.p.theta, m.p.dt);
         mac_threshold(m.p.theta, &mp[i].mid, &mp[i].tie);
         if (!(m.p.eps2 > 0.0f)) b->all_soft = false;
+        if (m.n >= kGroupMin) b->grouped = true;
     }
     if (S && is_octree_solver(b->solver))
         if (int r = ensure_octree(b)) return r;
@@ -321,6 +325,12 @@ void enqueue_pass_octree(nbg_batch *b) {
     wa.nt = n;
     wa.targets = b->bodies;
     wa.perm = b->idx;
+    if (b->grouped) {
+        uint32_t *perm = (uint32_t *)b->keys_alt;  // free once the nodes are built
+        launch_group_targets_forest(b->bodies, b->idx, n, b->sys_first, S, ob.targets, perm, s);
+        wa.targets = ob.targets;
+        wa.perm = perm;
+    }
     wa.nodes = nullptr;
     wa.onodes = ob.nodes;
     wa.levels = b->max_levels;
@@ -379,6 +389,13 @@ void enqueue_pass(nbg_batch *b) {
     wa.nt = n;
     wa.targets = b->bodies;
     wa.perm = b->idx;
+    if (b->grouped) {
+        // the summaries' queues and the sort's other half are free by now
+        float4 *targets = (float4 *)b->glist;
+        launch_group_targets_forest(b->bodies, b->idx, n, b->sys_first, S, targets, b->idx_alt, s);
+        wa.targets = targets;
+        wa.perm = b->idx_alt;
+    }
     wa.nodes = b->nodes;
     wa.onodes = nullptr;
     wa.levels = 0;

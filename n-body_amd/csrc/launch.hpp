@@ -136,6 +136,7 @@ inline int64_t octree_capacity(int64_t n, int leaf, int max_depth) {
 // Work buffers of the octree build (capacity `cap` nodes, n bodies).
 struct OctBuffers {
     int64_t cap = 0, n = 0;
+    float4 *targets = nullptr;  // forests: the walk's targets in their order
     uint64_t *key_hi = nullptr, *key_lo = nullptr, *lo_sorted = nullptr;  // n each
     uint32_t *nown = nullptr;      // n: nodes whose range starts at a position
     uint32_t *nbase = nullptr;     // n: exclusive scan of nown (pre-order node ids)
@@ -364,6 +365,17 @@ struct WalkArgs {
     float *split_part_f = nullptr;
     int64_t split_stride = 0;
 };
+
+// Walks of systems from this size on take their targets in compact groups
+// (targets.hip).  Below, the pass that forms them costs what it saves; walk
+// and pass, us, without / with: octree 80,000 bodies 246 / 278, 131,000 340 /
+// 360, 160,000 409 / 387; linear BVH 64,000 438 / 442, 131,000 794 / 784.
+constexpr int64_t kGroupMin = 160000;
+void launch_group_targets(const float4 *bodies, const uint32_t *perm, int64_t n, float4 *out, uint32_t *out_perm,
+                          hipStream_t s);
+// A forest's: systems below kGroupMin keep their order.
+void launch_group_targets_forest(const float4 *bodies, const uint32_t *perm, int64_t n, const int64_t *sys_first,
+                                 int nsys, float4 *out, uint32_t *out_perm, hipStream_t s);
 
 // ORDERED waves per 16 targets for a walk by frames of `groups` groups of 64
 // targets, 1: none.  Measured, walk us at n bodies, theta 0.5, leaf 16:
