@@ -137,6 +137,8 @@ int nbg_sys_update_accelerations(nbg_sys *sys, float *ax, float *ay, float *az);
 /* Copies the accelerations of the last force pass out (Acceleration component,
  * Physics/Acceleration.h:16-42). */
 int nbg_sys_get_accelerations(nbg_sys *sys, float *ax, float *ay, float *az);
+/* The same, interleaved: axyz holds 3 n floats, body by body. */
+int nbg_sys_get_accelerations_xyz(nbg_sys *sys, float *axyz);
 
 /* Accelerations at nt passive points (bodies without Mass): the reference
  * builds its tree from the actives, view<const Position, const Mass>, and walks
@@ -316,6 +318,9 @@ int nbg_batch_info(nbg_batch *b, int32_t *nsys, int64_t *nbodies);
  * those of the last pass and need a pass since the last membership change. */
 int nbg_batch_get(nbg_batch *b, int32_t id, float *x, float *y, float *z, float *vx, float *vy, float *vz,
                   float *ax, float *ay, float *az);
+/* The same with the accelerations interleaved (3 n floats, may be NULL). */
+int nbg_batch_get_xyz(nbg_batch *b, int32_t id, float *x, float *y, float *z, float *vx, float *vy, float *vz,
+                      float *axyz);
 
 /* Non-finite guard (no reference counterpart: the reference lets NaN
  * propagate): finds the systems whose positions or velocities hold a NaN or

@@ -39,14 +39,14 @@ EXPORTS = (
     "nbg_params_default", "nbg_last_error", "nbg_version", "nbg_device_count",
     "nbg_ctx_create", "nbg_ctx_destroy", "nbg_sys_create", "nbg_sys_destroy",
     "nbg_sys_set_params", "nbg_sys_get_params", "nbg_sys_set_state", "nbg_sys_get_state",
-    "nbg_sys_update_accelerations", "nbg_sys_get_accelerations", "nbg_sys_accelerations_at", "nbg_sys_accelerations_at_noalloc", "nbg_sys_step",
+    "nbg_sys_update_accelerations", "nbg_sys_get_accelerations", "nbg_sys_get_accelerations_xyz", "nbg_sys_accelerations_at", "nbg_sys_accelerations_at_noalloc", "nbg_sys_step",
     "nbg_sys_synchronize", "nbg_sys_counts", "nbg_sys_counts4", "nbg_sys_enable_counts", "nbg_sys_enable_walk_stats",
     "nbg_sys_walk_stats", "nbg_sys_set_walk_split",
     "nbg_sys_enable_timing", "nbg_sys_phase_times",
     "nbg_sys_debug_bbox", "nbg_sys_debug_order", "nbg_sys_debug_tree", "nbg_sys_debug_quads", "nbg_direct_f64",
     "nbg_sys_potential_f64", "nbg_generate_plummer", "nbg_generate_cube",
     "nbg_batch_bytes", "nbg_batch_create", "nbg_batch_destroy", "nbg_batch_add", "nbg_batch_remove",
-    "nbg_batch_set_params", "nbg_batch_info", "nbg_batch_get", "nbg_batch_update_accelerations", "nbg_batch_step",
+    "nbg_batch_set_params", "nbg_batch_info", "nbg_batch_get", "nbg_batch_get_xyz", "nbg_batch_update_accelerations", "nbg_batch_step",
     "nbg_batch_synchronize", "nbg_batch_counts", "nbg_batch_enable_counts", "nbg_batch_use_graph",
     "nbg_batch_autotune", "nbg_batch_autotune_grid", "nbg_batch_set_targets_per_lane", "nbg_batch_set_walk_split", "nbg_batch_nonfinite",
     "nbg_scenario_load_json", "nbg_scenario_load_tipsy", "nbg_scenario_count", "nbg_scenario_get", "nbg_scenario_free",
@@ -113,6 +113,7 @@ def lib() -> ctypes.CDLL:
             "nbg_sys_get_state": (ctypes.c_int, [_vp] + [_f32p] * 6),
             "nbg_sys_update_accelerations": (ctypes.c_int, [_vp] + [_f32p] * 3),
             "nbg_sys_get_accelerations": (ctypes.c_int, [_vp] + [_f32p] * 3),
+            "nbg_sys_get_accelerations_xyz": (ctypes.c_int, [_vp, _f32p]),
             "nbg_sys_accelerations_at": (ctypes.c_int, [_vp, ctypes.c_int64] + [_f32p] * 6),
             "nbg_sys_accelerations_at_noalloc": (ctypes.c_int, [_vp, ctypes.c_int64] + [_f32p] * 6),
             "nbg_batch_bytes": (ctypes.c_int64, [ctypes.c_int64, ctypes.c_int32]),
@@ -125,6 +126,7 @@ def lib() -> ctypes.CDLL:
             "nbg_batch_set_params": (ctypes.c_int, [_vp, ctypes.c_int32, ctypes.POINTER(Params)]),
             "nbg_batch_info": (ctypes.c_int, [_vp, ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_int64)]),
             "nbg_batch_get": (ctypes.c_int, [_vp, ctypes.c_int32] + [_f32p] * 9),
+            "nbg_batch_get_xyz": (ctypes.c_int, [_vp, ctypes.c_int32] + [_f32p] * 7),
             "nbg_batch_update_accelerations": (ctypes.c_int, [_vp]),
             "nbg_batch_nonfinite": (ctypes.c_int, [_vp, ctypes.POINTER(ctypes.c_int32), ctypes.c_int32,
                                                    ctypes.POINTER(ctypes.c_int32)]),
@@ -330,14 +332,13 @@ class System:
         return out
 
     def update_accelerations(self) -> np.ndarray:
-        a = [np.zeros(self.n, np.float32) for _ in range(3)]
-        _check(lib().nbg_sys_update_accelerations(self.handle, *[_ptr(v) for v in a]))
-        return np.stack(a, axis=1)
+        _check(lib().nbg_sys_update_accelerations(self.handle, None, None, None))
+        return self.accelerations()
 
     def accelerations(self) -> np.ndarray:
-        a = [np.zeros(self.n, np.float32) for _ in range(3)]
-        _check(lib().nbg_sys_get_accelerations(self.handle, *[_ptr(v) for v in a]))
-        return np.stack(a, axis=1)
+        a = np.empty((self.n, 3), np.float32)
+        _check(lib().nbg_sys_get_accelerations_xyz(self.handle, _ptr(a)))
+        return a
 
     def accelerations_at(self, tx, ty, tz) -> np.ndarray:
         """Accelerations at passive points (bodies without Mass) from the
@@ -492,10 +493,10 @@ class Batch:
     def get(self, sid: int, accelerations: bool = False):
         n = self._n[sid]
         out = Bodies.empty(n)
-        acc = [np.zeros(n, np.float32) for _ in range(3)] if accelerations else [None] * 3
-        _check(lib().nbg_batch_get(self.handle, sid, *[_ptr(v) for v in (out.x, out.y, out.z, out.vx, out.vy, out.vz)],
-                                   *[_ptr(v) if v is not None else None for v in acc]))
-        return (out, np.stack(acc, axis=1)) if accelerations else out
+        acc = np.empty((n, 3), np.float32) if accelerations else None
+        _check(lib().nbg_batch_get_xyz(self.handle, sid, *[_ptr(v) for v in (out.x, out.y, out.z, out.vx, out.vy, out.vz)],
+                                       _ptr(acc)))
+        return (out, acc) if accelerations else out
 
     def nonfinite(self):
         """Ids of the systems whose positions or velocities hold NaN or inf."""

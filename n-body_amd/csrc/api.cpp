@@ -13,6 +13,7 @@
 
 #include "../../include/nbg.h"
 #include "host_util.hpp"
+#include "transfer.hpp"
 #include "launch.hpp"
 
 using namespace nbg;
@@ -499,6 +500,19 @@ int report_device_error(nbg_sys *s, uint32_t err) {
     return fail(NBG_ERR_DEVICE, "device error flag set");
 }
 
+// Device rows d to the host arrays h that are not null.
+int copy_rows(nbg_sys *s, float *const *h, float *const *d, int k) {
+    NBG_HIP(hipStreamSynchronize(s->stream));
+    RowSet R;
+    float *dst[10];
+    for (int j = 0; j < k; ++j)
+        if (h[j]) {
+            dst[R.k] = h[j];
+            R.row[R.k++] = d[j];
+        }
+    return rows_out(s->ctx, s->stream, R, dst, s->n);
+}
+
 int sync_and_check(nbg_sys *s) {
     NBG_HIP(hipStreamSynchronize(s->stream));
     uint32_t err = 0;
@@ -703,11 +717,16 @@ int nbg_ctx_create(int device, nbg_ctx **out) {
     nbg_ctx *ctx = new nbg_ctx;
     ctx->device = device;
     ctx->noalloc_scratch = scr;
+    ctx->staging = new Staging;
     *out = ctx;
     return NBG_OK;
 }
 
 int nbg_ctx_destroy(nbg_ctx *ctx) {
+    if (ctx) {
+        ctx->staging->release();
+        delete ctx->staging;
+    }
     delete ctx;
     return NBG_OK;
 }
@@ -795,20 +814,10 @@ int nbg_sys_set_state(nbg_sys *s, const float *x, const float *y, const float *z
                       const float *vy, const float *vz) {
     if (!s || !x || !y || !z || !m) return fail(NBG_ERR_ARG, "positions and masses are required");
     DeviceGuard g(s->ctx->device);
-    const size_t b = (size_t)s->n * sizeof(float);
-    if (s->n > 0) {
-        NBG_HIP(hipMemcpyAsync(s->x, x, b, hipMemcpyHostToDevice, s->stream));
-        NBG_HIP(hipMemcpyAsync(s->y, y, b, hipMemcpyHostToDevice, s->stream));
-        NBG_HIP(hipMemcpyAsync(s->z, z, b, hipMemcpyHostToDevice, s->stream));
-        NBG_HIP(hipMemcpyAsync(s->m, m, b, hipMemcpyHostToDevice, s->stream));
-        float *dv[3] = {s->vx, s->vy, s->vz};
-        const float *hv[3] = {vx, vy, vz};
-        for (int d = 0; d < 3; ++d) {
-            if (hv[d]) NBG_HIP(hipMemcpyAsync(dv[d], hv[d], b, hipMemcpyHostToDevice, s->stream));
-            else launch_fill_u32((uint32_t *)dv[d], 0u, s->n, s->stream);
-        }
-        NBG_HIP(hipStreamSynchronize(s->stream));
-    }
+    const RowSet R{{s->x, s->y, s->z, s->m, s->vx, s->vy, s->vz}, 7, false};
+    const float *src[7] = {x, y, z, m, vx, vy, vz};
+    NBG_HIP(hipStreamSynchronize(s->stream));
+    if (int r = rows_in(s->ctx, s->stream, R, src, s->n)) return r;
     s->have_state = true;
     s->have_forces = false;
     s->tree_valid = false;
@@ -818,13 +827,9 @@ int nbg_sys_set_state(nbg_sys *s, const float *x, const float *y, const float *z
 int nbg_sys_get_state(nbg_sys *s, float *x, float *y, float *z, float *vx, float *vy, float *vz) {
     if (!s) return fail(NBG_ERR_ARG, "sys is NULL");
     DeviceGuard g(s->ctx->device);
-    const size_t b = (size_t)s->n * sizeof(float);
     float *h[6] = {x, y, z, vx, vy, vz};
     float *d[6] = {s->x, s->y, s->z, s->vx, s->vy, s->vz};
-    NBG_HIP(hipStreamSynchronize(s->stream));
-    for (int i = 0; i < 6; ++i)
-        if (h[i] && s->n > 0) NBG_HIP(hipMemcpy(h[i], d[i], b, hipMemcpyDeviceToHost));
-    return NBG_OK;
+    return copy_rows(s, h, d, 6);
 }
 
 int nbg_sys_update_accelerations(nbg_sys *s, float *ax, float *ay, float *az) {
@@ -843,14 +848,17 @@ int nbg_sys_get_accelerations(nbg_sys *s, float *ax, float *ay, float *az) {
     if (!s) return fail(NBG_ERR_ARG, "sys is NULL");
     if (!s->have_forces) return fail(NBG_ERR_STATE, "no force pass has run");
     DeviceGuard g(s->ctx->device);
+    float *h[3] = {ax, ay, az};
+    float *d[3] = {s->ax, s->ay, s->az};
+    return copy_rows(s, h, d, 3);
+}
+
+int nbg_sys_get_accelerations_xyz(nbg_sys *s, float *axyz) {
+    if (!s || !axyz) return fail(NBG_ERR_ARG, "sys or axyz is NULL");
+    if (!s->have_forces) return fail(NBG_ERR_STATE, "no force pass has run");
+    DeviceGuard g(s->ctx->device);
     NBG_HIP(hipStreamSynchronize(s->stream));
-    const size_t b = (size_t)s->n * sizeof(float);
-    if (s->n > 0) {
-        if (ax) NBG_HIP(hipMemcpy(ax, s->ax, b, hipMemcpyDeviceToHost));
-        if (ay) NBG_HIP(hipMemcpy(ay, s->ay, b, hipMemcpyDeviceToHost));
-        if (az) NBG_HIP(hipMemcpy(az, s->az, b, hipMemcpyDeviceToHost));
-    }
-    return NBG_OK;
+    return rows_out(s->ctx, s->stream, RowSet{{s->ax, s->ay, s->az}, 3, true}, &axyz, s->n);
 }
 
 int nbg_sys_accelerations_at(nbg_sys *s, int64_t nt, const float *tx, const float *ty, const float *tz, float *ax,

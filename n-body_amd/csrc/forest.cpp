@@ -20,6 +20,7 @@
 
 #include "../../include/nbg.h"
 #include "host_util.hpp"
+#include "transfer.hpp"
 #include "launch.hpp"
 
 using namespace nbg;
@@ -536,14 +537,11 @@ int nbg_batch_add(nbg_batch *b, const nbg_params *p, int64_t n, const float *x, 
     if (int r = check_member_solver(b, p, nullptr)) return r;
     hipStream_t s = b->stream;
     NBG_HIP(hipStreamSynchronize(s));
-    const size_t bytes = (size_t)n * 4;
-    const float *h[7] = {x, y, z, m, vx, vy, vz};
-    for (int k = 0; k < 7; ++k) {
-        if (h[k]) NBG_HIP(hipMemcpyAsync(b->st[k] + used, h[k], bytes, hipMemcpyHostToDevice, s));
-        else launch_fill_u32((uint32_t *)(b->st[k] + used), 0u, n, s);
-    }
-    for (int k = 7; k < 10; ++k) launch_fill_u32((uint32_t *)(b->st[k] + used), 0u, n, s);
-    NBG_HIP(hipStreamSynchronize(s));
+    const float *h[10] = {x, y, z, m, vx, vy, vz, nullptr, nullptr, nullptr};
+    RowSet R;
+    R.k = 10;
+    for (int k = 0; k < 10; ++k) R.row[k] = b->st[k] + used;
+    if (int r = rows_in(b->ctx, s, R, h, n)) return r;
     Member mm;
     mm.id = b->next_id++;
     mm.n = n;
@@ -610,15 +608,18 @@ int nbg_batch_set_params(nbg_batch *b, int32_t id, const nbg_params *p) {
     return NBG_OK;
 }
 
-int nbg_batch_get(nbg_batch *b, int32_t id, float *x, float *y, float *z, float *vx, float *vy, float *vz, float *ax,
-                  float *ay, float *az) {
+// nbg_batch_get's rows; xyz: accelerations interleaved into h[6].
+static int batch_rows(nbg_batch *b, int32_t id, float *const *h, bool xyz) {
     if (!b) return fail(NBG_ERR_ARG, "batch is NULL");
     Member *mm = find(b, id);
     if (!mm) return fail(NBG_ERR_ARG, "unknown system id");
     DeviceGuard g(b->ctx->device);
-    if (int r = sync_check(b)) return r;
-    if ((ax || ay || az) && !b->have_forces) return fail(NBG_ERR_STATE, "no force pass since the last change");
-    float *h[9] = {x, y, z, vx, vy, vz, ax, ay, az};
+    NBG_HIP(hipStreamSynchronize(b->stream));
+    const bool forces = xyz ? h[6] != nullptr : h[6] || h[7] || h[8];
+    if (forces && !b->have_forces) {
+        if (int r = sync_check(b)) return r;
+        return fail(NBG_ERR_STATE, "no force pass since the last change");
+    }
     const int map[9] = {0, 1, 2, 4, 5, 6, 7, 8, 9};
     // offsets may be stale if membership changed after the last pass
     int64_t first = 0;
@@ -626,9 +627,33 @@ int nbg_batch_get(nbg_batch *b, int32_t id, float *x, float *y, float *z, float 
         if (o.id == id) break;
         first += o.n;
     }
-    for (int k = 0; k < 9; ++k)
-        if (h[k]) NBG_HIP(hipMemcpy(h[k], b->st[map[k]] + first, (size_t)mm->n * 4, hipMemcpyDeviceToHost));
-    return NBG_OK;
+    RowSet R;
+    float *dst[9];
+    for (int k = 0; k < (xyz ? 6 : 9); ++k)
+        if (h[k]) {
+            dst[R.k] = h[k];
+            R.row[R.k++] = b->st[map[k]] + first;
+        }
+    if (xyz && h[6]) {
+        R.xyz = true;
+        dst[R.k] = h[6];
+        for (int c = 0; c < 3; ++c) R.row[R.k++] = b->st[7 + c] + first;
+    }
+    uint32_t err = 0;
+    if (int r = rows_out(b->ctx, b->stream, R, dst, mm->n, b->err_word(), &err)) return r;
+    return err ? sync_check(b) : NBG_OK;
+}
+
+int nbg_batch_get(nbg_batch *b, int32_t id, float *x, float *y, float *z, float *vx, float *vy, float *vz, float *ax,
+                  float *ay, float *az) {
+    float *h[9] = {x, y, z, vx, vy, vz, ax, ay, az};
+    return batch_rows(b, id, h, false);
+}
+
+int nbg_batch_get_xyz(nbg_batch *b, int32_t id, float *x, float *y, float *z, float *vx, float *vy, float *vz,
+                      float *axyz) {
+    float *h[7] = {x, y, z, vx, vy, vz, axyz};
+    return batch_rows(b, id, h, true);
 }
 
 int nbg_batch_update_accelerations(nbg_batch *b) {

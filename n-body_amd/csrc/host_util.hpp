@@ -44,9 +44,14 @@ struct DeviceGuard {
 
 }  // namespace nbg
 
+namespace nbg {
+struct Staging;
+}
+
 // A context binds one GPU.
 struct nbg_ctx {
     int device = 0;
+    nbg::Staging *staging = nullptr;  // pinned memory for host copies
     // this device's copy of the allocation-free passive-point scratch
     // (looked up with hipGetSymbolAddress at nbg_ctx_create)
     void *noalloc_scratch = nullptr;

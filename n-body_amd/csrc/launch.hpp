@@ -377,6 +377,21 @@ void launch_group_targets(const float4 *bodies, const uint32_t *perm, int64_t n,
 void launch_group_targets_forest(const float4 *bodies, const uint32_t *perm, int64_t n, const int64_t *sys_first,
                                  int nsys, float4 *out, uint32_t *out_perm, hipStream_t s);
 
+// Rows of floats that are copied to or from the host together; xyz: the last
+// three go out interleaved.
+struct RowSet {
+    float *row[10] = {};
+    int k = 0;
+    bool xyz = false;
+};
+// Elements i0 .. i0 + cnt - 1 of every row to words 0 .. k * stride - 1 (pinned
+// host memory, row j from j * stride on; stride a multiple of 4), and *err
+// (may be null) to *err_out.
+void launch_rows_out(const RowSet &R, int64_t i0, int cnt, int stride, float *words, const uint32_t *err,
+                     uint32_t *err_out, hipStream_t s);
+// The other way; rows in `absent` are cleared.
+void launch_rows_in(const RowSet &R, int cnt, int stride, const float *words, uint32_t absent, hipStream_t s);
+
 // ORDERED waves per 16 targets for a walk by frames of `groups` groups of 64
 // targets, 1: none.  Measured, walk us at n bodies, theta 0.5, leaf 16:
 // octree, 8 / 16 waves / recursion (the split that was here before): 1,000 59

@@ -335,6 +335,61 @@ void launch_pack(const float *x, const float *y, const float *z, const float *m,
     hipLaunchKernelGGL(k_pack, dim3((unsigned)blocks), dim3(256), 0, s, x, y, z, m, n, out);
 }
 
+// Four consecutive words a thread: 16-byte accesses over the bus.
+__global__ __launch_bounds__(256) void k_rows_out(RowSet R, int64_t i0, int cnt, int stride, float4 *__restrict__ words,
+                                                  const uint32_t *__restrict__ err, uint32_t *__restrict__ err_out) {
+    const int per = stride / 4, total = R.k * per;
+    const int t0 = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t0 == 0 && err) *err_out = *err;
+    const int whole = R.xyz ? R.k - 3 : R.k;
+    for (int t = t0; t < total; t += gridDim.x * blockDim.x) {
+        const int j = t / per, q = (t - j * per) * 4;
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            int row = j, i = q + e;
+            if (j >= whole) {
+                const int w = (j - whole) * stride + q + e;
+                i = w / 3;
+                row = whole + (w - 3 * i);
+            }
+            v[e] = i < cnt ? R.row[row][i0 + i] : 0.0f;
+        }
+        words[t] = make_float4(v[0], v[1], v[2], v[3]);
+    }
+}
+
+__global__ __launch_bounds__(256) void k_rows_in(RowSet R, int cnt, int stride, const float4 *__restrict__ words,
+                                                 uint32_t absent) {
+    const int per = stride / 4, total = R.k * per;
+    for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < total; t += gridDim.x * blockDim.x) {
+        const int j = t / per, q = (t - j * per) * 4;
+        float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (!((absent >> j) & 1u)) v = words[t];
+        float *const r = R.row[j] + q;
+        if (q < cnt) r[0] = v.x;
+        if (q + 1 < cnt) r[1] = v.y;
+        if (q + 2 < cnt) r[2] = v.z;
+        if (q + 3 < cnt) r[3] = v.w;
+    }
+}
+
+static unsigned rows_blocks(const RowSet &R, int stride) {
+    const int blocks = (R.k * (stride / 4) + 255) / 256;
+    return (unsigned)(blocks < 1024 ? blocks : 1024);
+}
+
+void launch_rows_out(const RowSet &R, int64_t i0, int cnt, int stride, float *words, const uint32_t *err,
+                     uint32_t *err_out, hipStream_t s) {
+    hipLaunchKernelGGL(k_rows_out, dim3(rows_blocks(R, stride)), dim3(256), 0, s, R, i0, cnt, stride, (float4 *)words,
+                       err, err_out);
+}
+
+void launch_rows_in(const RowSet &R, int cnt, int stride, const float *words, uint32_t absent, hipStream_t s) {
+    hipLaunchKernelGGL(k_rows_in, dim3(rows_blocks(R, stride)), dim3(256), 0, s, R, cnt, stride, (const float4 *)words,
+                       absent);
+}
+
 int64_t potential_waves(int64_t n) { return (n + kWave - 1) / kWave; }
 
 void launch_pack_f64(const float *x, const float *y, const float *z, const float *m, int64_t n, double4 *out,
