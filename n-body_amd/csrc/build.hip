@@ -1206,17 +1206,16 @@ void launch_lbvh_summaries(const float4 *bodies, int64_t n, NodeRec *nodes, cons
 // that span systems always split, the radix tree over the concatenation holds
 // each system's reference tree as the subtree whose range is that system.
 
-__global__ __launch_bounds__(256) void k_seg_bbox(const float *__restrict__ x, const float *__restrict__ y,
-                                                  const float *__restrict__ z, const int64_t *__restrict__ sys_first,
-                                                  float *bbox6) {
-    const int sys = blockIdx.x;
-    const int64_t lo = sys_first[sys], hi = sys_first[sys + 1];
-    float mn[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, mx[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
-    for (int64_t i = lo + threadIdx.x; i < hi; i += blockDim.x) {
-        float v[3] = {x[i], y[i], z[i]};
-#pragma unroll
-        for (int d = 0; d < 3; ++d) { mn[d] = fmin_ref(mn[d], v[d]); mx[d] = fmax_ref(mx[d], v[d]); }
-    }
+// Boxes of the systems, a workgroup per kSegPart bodies or less of one: the
+// workgroups of system i are those from sys_first[i] / kSegPart + i on, of
+// which some stay empty.  A system of several parts leaves their boxes in
+// `part` (24 bytes for every kSegPart / 4 positions: parts start at least
+// kSegPart / 2 apart) for k_seg_fold.  With one workgroup a system 128
+// members of 256 to 65,536 bodies took 72 us and one of 239,000 took 229; so
+// the former take 16, and 5 to fold.
+constexpr int kSegPart = 8192;
+
+__device__ __forceinline__ void seg_reduce(float (&mn)[3], float (&mx)[3]) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1)
 #pragma unroll
@@ -1224,6 +1223,33 @@ __global__ __launch_bounds__(256) void k_seg_bbox(const float *__restrict__ x, c
             mn[d] = fmin_ref(mn[d], __shfl_xor(mn[d], o, kWave));
             mx[d] = fmax_ref(mx[d], __shfl_xor(mx[d], o, kWave));
         }
+}
+__device__ __forceinline__ int64_t seg_parts(int64_t n) { return (n + kSegPart - 1) / kSegPart; }
+// First position of part j in a system of n bodies: every part of several has
+// kSegPart / 2 bodies or more.
+__device__ __forceinline__ int64_t seg_start(int64_t n, int64_t parts, int64_t j) { return n * j / parts; }
+
+__global__ __launch_bounds__(256) void k_seg_bbox(const float *__restrict__ x, const float *__restrict__ y,
+                                                  const float *__restrict__ z, int nsys,
+                                                  const int64_t *__restrict__ sys_first, float *bbox6, float *part) {
+    const int64_t block = blockIdx.x;
+    int sys = 0, end = nsys;
+    while (end - sys > 1) {
+        const int mid = (sys + end) >> 1;
+        if (sys_first[mid] / kSegPart + mid <= block) sys = mid;
+        else end = mid;
+    }
+    const int64_t first = sys_first[sys], last = sys_first[sys + 1];
+    const int64_t n = last - first, parts = n > 0 ? seg_parts(n) : 1, j = block - (first / kSegPart + sys);
+    if (j >= parts) return;  // the whole workgroup
+    const int64_t lo = first + seg_start(n, parts, j), hi = first + seg_start(n, parts, j + 1);
+    float mn[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, mx[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
+    for (int64_t i = lo + threadIdx.x; i < hi; i += blockDim.x) {
+        float v[3] = {x[i], y[i], z[i]};
+#pragma unroll
+        for (int d = 0; d < 3; ++d) { mn[d] = fmin_ref(mn[d], v[d]); mx[d] = fmax_ref(mx[d], v[d]); }
+    }
+    seg_reduce(mn, mx);
     __shared__ float s_part[4][6];
     const int w = threadIdx.x / kWave;
     if (lane_id() == 0)
@@ -1234,8 +1260,27 @@ __global__ __launch_bounds__(256) void k_seg_bbox(const float *__restrict__ x, c
         for (int d = 0; d < 6; ++d) r[d] = s_part[0][d];
         for (int ww = 1; ww < 4; ++ww)
             for (int d = 0; d < 3; ++d) { r[d] = fmin_ref(r[d], s_part[ww][d]); r[3 + d] = fmax_ref(r[3 + d], s_part[ww][3 + d]); }
-        for (int d = 0; d < 6; ++d) bbox6[sys * 6 + d] = r[d];
+        float *const out = parts > 1 ? part + 6 * (lo / (kSegPart / 4)) : bbox6 + 6 * (int64_t)sys;
+        for (int d = 0; d < 6; ++d) out[d] = r[d];
     }
+}
+
+// The boxes of the systems of several parts, a wave each.
+__global__ __launch_bounds__(64) void k_seg_fold(const int64_t *__restrict__ sys_first, const float *__restrict__ part,
+                                                 float *bbox6) {
+    const int sys = blockIdx.x;
+    const int64_t first = sys_first[sys], n = sys_first[sys + 1] - first, parts = seg_parts(n);
+    if (parts <= 1) return;
+    float mn[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, mx[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
+    for (int64_t j = threadIdx.x; j < parts; j += kWave) {
+        const int64_t lo = first + seg_start(n, parts, j);
+        const float *const r = part + 6 * (lo / (kSegPart / 4));
+#pragma unroll
+        for (int d = 0; d < 3; ++d) { mn[d] = fmin_ref(mn[d], r[d]); mx[d] = fmax_ref(mx[d], r[3 + d]); }
+    }
+    seg_reduce(mn, mx);
+    if (threadIdx.x == 0)
+        for (int d = 0; d < 3; ++d) { bbox6[6 * (int64_t)sys + d] = mn[d]; bbox6[6 * (int64_t)sys + 3 + d] = mx[d]; }
 }
 
 __global__ __launch_bounds__(256) void k_forest_keys(const float *__restrict__ x, const float *__restrict__ y,
@@ -1281,7 +1326,8 @@ __global__ __launch_bounds__(256) void k_forest_roots(const NodeRec *__restrict_
 }
 
 void launch_forest_build(const float *x, const float *y, const float *z, int64_t n, int nsys,
-                         const int64_t *sys_first, const uint32_t *bsys, float *bbox6, uint64_t *keys, uint32_t *idx,
+                         const int64_t *sys_first, int64_t largest, const uint32_t *bsys, float *bbox6,
+                         uint64_t *keys, uint32_t *idx,
                          uint64_t *keys_alt, uint32_t *idx_alt, uint32_t *sort_status, FillSet &fills, uint32_t *err,
                          hipStream_t s) {
     if (n <= 0 || nsys <= 0) return;
@@ -1289,7 +1335,7 @@ void launch_forest_build(const float *x, const float *y, const float *z, int64_t
     while ((1ll << sbits) < nsys) ++sbits;
     const SortPlan plan = sort_plan(n, 30 + sbits, false);
     fills.add(sort_status, sort_clear_words(n, plan));
-    hipLaunchKernelGGL(k_seg_bbox, dim3((unsigned)nsys), dim3(256), 0, s, x, y, z, sys_first, bbox6);
+    launch_seg_bbox(x, y, z, n, nsys, sys_first, largest, bbox6, (float *)keys, s);
     launch_fills(fills, s);
     int64_t blocks = (n + 255) / 256;
     if (blocks > 2048) blocks = 2048;
@@ -1299,10 +1345,12 @@ void launch_forest_build(const float *x, const float *y, const float *z, int64_t
     launch_sort(keys, idx, keys_alt, idx_alt, n, 64, plan, sort_status, err, s);
 }
 
-void launch_seg_bbox(const float *x, const float *y, const float *z, int nsys, const int64_t *sys_first,
-                     float *bbox6, hipStream_t s) {
+void launch_seg_bbox(const float *x, const float *y, const float *z, int64_t n, int nsys, const int64_t *sys_first,
+                     int64_t largest, float *bbox6, float *part, hipStream_t s) {
     if (nsys <= 0) return;
-    hipLaunchKernelGGL(k_seg_bbox, dim3((unsigned)nsys), dim3(256), 0, s, x, y, z, sys_first, bbox6);
+    hipLaunchKernelGGL(k_seg_bbox, dim3((unsigned)(n / kSegPart + nsys)), dim3(256), 0, s, x, y, z, nsys, sys_first,
+                       bbox6, part);
+    if (largest > kSegPart) hipLaunchKernelGGL(k_seg_fold, dim3((unsigned)nsys), dim3(64), 0, s, sys_first, part, bbox6);
 }
 
 void launch_forest_roots(const NodeRec *nodes, const uint32_t *node_count, int64_t max_nodes, const uint64_t *keys,

@@ -95,6 +95,7 @@ struct nbg_batch {
     // targets per lane asked for (the autotuner's bodies-per-wavefront
     // choice): a hint that the present walks do not need
     int32_t tpl = 1;
+    int64_t largest = 0;    // bodies of the largest member
     bool grouped = false;   // a member takes its targets in groups (kGroupMin)
     int32_t split_req = 0;  // waves per group of the FAST walk: 0 = by size
     float *x() { return st[0]; }
@@ -256,6 +257,7 @@ int upload_tables(nbg_batch *b) {
     int64_t off = 0, w = 0;
     b->all_soft = true;
     b->grouped = false;
+    b->largest = 0;
     b->max_levels = 0;
     if (S) b->solver = b->sys[0].p.solver;
     const int64_t width = 64;  // targets per group
@@ -274,6 +276,7 @@ int upload_tables(nbg_batch *b) {
         mac_threshold(m.p.theta, &mp[i].mid, &mp[i].tie);
         if (!(m.p.eps2 > 0.0f)) b->all_soft = false;
         if (m.n >= kGroupMin) b->grouped = true;
+        if (m.n > b->largest) b->largest = m.n;
     }
     if (S && is_octree_solver(b->solver))
         if (int r = ensure_octree(b)) return r;
@@ -312,7 +315,7 @@ void enqueue_pass_octree(nbg_batch *b) {
     oct_fills(fills, ob, n, b->leaf_start);
     fills.add(b->misc + 4, 12);
     launch_fills(fills, s);
-    launch_seg_bbox(b->x(), b->y(), b->z(), S, b->sys_first, b->bbox6, s);
+    launch_seg_bbox(b->x(), b->y(), b->z(), n, S, b->sys_first, b->largest, b->bbox6, (float *)b->keys, s);
     launch_octree_forest_build(b->x(), b->y(), b->z(), n, S, b->bsys, b->bbox6, b->lv_tab, b->max_levels, ob,
                                b->keys, b->idx, b->keys_alt, b->idx_alt, b->sort_status, b->err_word(), s);
     launch_octree_forest_topology(n, S, b->bbox6, b->sys_prm, b->lv_tab, b->leaf_tab, b->sys_first, b->max_levels,
@@ -375,7 +378,7 @@ void enqueue_pass(nbg_batch *b) {
     FillSet fills;
     lbvh_fills(fills, n, b->leaf_start, b->scan_ws, b->flags);
     fills.add(b->misc + 4, 12);
-    launch_forest_build(b->x(), b->y(), b->z(), n, S, b->sys_first, b->bsys, b->bbox6, b->keys, b->idx, b->keys_alt,
+    launch_forest_build(b->x(), b->y(), b->z(), n, S, b->sys_first, b->largest, b->bsys, b->bbox6, b->keys, b->idx, b->keys_alt,
                         b->idx_alt, b->sort_status, fills, b->err_word(), s);
     launch_lbvh_topology(b->keys, 63, n, 0, b->kfirst, b->klast, b->kgamma, b->ksplit, b->krank, b->kparent,
                          b->scan_ws, b->nodes, b->leaf_start, b->node_count(), b->x(), b->y(), b->z(), b->m(), b->idx,

@@ -7,7 +7,7 @@
 
 namespace nbg {
 
-// Radix-sort geometry (onesweep): 256 threads x kSortItems keys per tile.
+// Radix-sort geometry (onesweep): 256 threads x sort_items(n) keys per tile.
 // Fewer keys a thread while more would leave the chip short of tiles: a pass
 // over u64 keys takes 6.7 us with 4 keys a thread and 11.0 with 16 at 10,000
 // keys, 16.8 with 8 and 18 with 16 at 500,000, 27 with 8 and 23 with 16 at
@@ -51,6 +51,10 @@ inline SortPlan sort_plan(int64_t n, int bits, bool lo) {
     while (((int64_t)1 << (need - 10)) < n) ++need;
     SortPlan p;
     p.passes = sort_passes(need) < full ? sort_passes(need) : full;
+    // A last pass costs what ranking the runs does, and no run can be long
+    // (73,000 bodies of a forest, 34-bit keys: cells of the cores hold
+    // hundreds, and sorting those runs took 2 ms, a pass takes 12 us).
+    if (p.passes + 1 == full && !lo) p.passes = full;
     p.shift = bits > 8 * p.passes ? bits - 8 * p.passes : 0;
     p.runs = p.shift > 0 || lo;
     // the last kernel reads the _alt buffers (runs), or the last pass writes the primary ones
@@ -208,9 +212,10 @@ void launch_octree_forest_topology(int64_t n, int nsys, const float *bbox6, cons
                                    const uint32_t *idx_alt, uint32_t *idx, int32_t *leaf_start, uint32_t *err,
                                    hipStream_t s);
 
-// Per-system bounding boxes (one workgroup per system).
-void launch_seg_bbox(const float *x, const float *y, const float *z, int nsys, const int64_t *sys_first,
-                     float *bbox6, hipStream_t s);
+// Per-system bounding boxes; part: scratch of 24 bytes for every 2,048 bodies
+// (used if the largest system has more than 8,192).
+void launch_seg_bbox(const float *x, const float *y, const float *z, int64_t n, int nsys, const int64_t *sys_first,
+                     int64_t largest, float *bbox6, float *part, hipStream_t s);
 
 void launch_octree_summaries(const float4 *bodies, int64_t n, OctBuffers &ob, const int32_t *leaf_start,
                              uint32_t *err, hipStream_t s, float4 *quad = nullptr);
@@ -295,7 +300,7 @@ void launch_lbvh_summaries(const float4 *bodies, int64_t n, NodeRec *nodes, cons
 // per-system bounding boxes (bbox6: 6 floats per system), keys, and one sort;
 // sets `fills` and the sort's words first.
 void launch_forest_build(const float *x, const float *y, const float *z, int64_t n, int nsys,
-                         const int64_t *sys_first, const uint32_t *bsys, float *bbox6, uint64_t *keys, uint32_t *idx,
+                         const int64_t *sys_first, int64_t largest, const uint32_t *bsys, float *bbox6, uint64_t *keys, uint32_t *idx,
                          uint64_t *keys_alt, uint32_t *idx_alt, uint32_t *sort_status, FillSet &fills, uint32_t *err,
                          hipStream_t s);
 // sys_root[s] = slot of the node whose range is exactly system s.
