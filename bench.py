@@ -247,7 +247,7 @@ def measure(nbg, ctx, b, args, solver, mode=None):
     flops = (FLOPS_PER_INTERACTION * pp + (FLOPS_PER_QUAD_NODE if quad else FLOPS_PER_INTERACTION) * npc
              + FLOPS_PER_LOCAL * (pn + nn))
     achieved = flops / (walk_ms * 1e-3) / 1e12
-    waves = max(1, (args.n + 63) // 64)
+    waves = max(1, (args.n + 15) // 16)  # the FAST tree walks' (16 targets each)
     # the traffic file keys the ORDERED walks' rows "<solver>-ordered"
     traffic = load_traffic().get(SOLVER_NAMES[solver] + ("" if mode == "fast" else "-ordered"))
     out = {
@@ -261,9 +261,9 @@ def measure(nbg, ctx, b, args, solver, mode=None):
         "interaction_counts": {"pp": pp, "np": npc, "pn": pn, "nn": nn},
         "walk_schedule": {
             "node_visits_per_wave": ws["node_visits"] / waves,
-            "lane_utilisation_nodes": ws["active_lanes"] / max(1, 64 * ws["node_visits"]),
+            "lane_utilisation_nodes": ws["active_lanes"] / max(1, 16 * ws["node_visits"]),
             "leaf_visits_per_wave": ws["leaf_visits"] / waves,
-            "lane_utilisation_leaves": ws["leaf_lanes"] / max(1, 64 * ws["leaf_visits"]),
+            "lane_utilisation_leaves": ws["leaf_lanes"] / max(1, 16 * ws["leaf_visits"]),
         } if not fmm and ws["node_visits"] else (ws if fmm else None),
         "roofline": {
             "bound": "valu",
