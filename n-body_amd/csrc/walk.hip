@@ -327,7 +327,7 @@ __global__ __launch_bounds__(64 * kOrderedWaves) void k_walk_lbvh_ordered(WalkAr
     __shared__ float s_ring_all[kOrderedWaves][kSaveRing * 3 * kWave];
 
     const int lane = lane_id(), wv = uniform_i32(threadIdx.x / kWave);
-    const WaveTask T = wave_task<FOREST>(a, (int64_t)xcd_block(blockIdx.x, gridDim.x) * kOrderedWaves + wv);
+    const WaveTask T = wave_task<FOREST>(a, (int64_t)walk_block<FOREST>() * kOrderedWaves + wv);
     const int64_t tgt = T.base + lane;
     const bool valid = tgt < T.end;
     const uint64_t vmask = __ballot(valid);
@@ -520,7 +520,7 @@ __global__ __launch_bounds__(64 * K) void k_walk_lbvh_ordered_frames(WalkArgs a)
 
     const int lane = lane_id(), wv = uniform_i32(threadIdx.x / kWave), bit = target_bit<true>();
     const int row = lane / kRowTargets;
-    const int64_t sub = xcd_block(blockIdx.x, gridDim.x);
+    const int64_t sub = walk_block<FOREST>();
     const WaveTask T = wave_task<FOREST>(a, sub / 4);
     const int64_t tgt = T.base + (sub % 4) * kRowTargets + bit;
     const bool valid = tgt < T.end;
@@ -865,7 +865,7 @@ __global__ __launch_bounds__(64 * kOrderedWaves) void k_walk_oct_ordered(WalkArg
     __shared__ int s_pos_all[kOrderedWaves][MAXL];  // next child index | next octant << 8
     __shared__ uint64_t s_mask_all[kOrderedWaves][MAXL];
     const int lane = lane_id(), wv = uniform_i32(threadIdx.x / kWave);
-    const WaveTask T = wave_task<FOREST>(a, (int64_t)xcd_block(blockIdx.x, gridDim.x) * kOrderedWaves + wv);
+    const WaveTask T = wave_task<FOREST>(a, (int64_t)walk_block<FOREST>() * kOrderedWaves + wv);
     const int64_t tgt = T.base + lane;
     const bool valid = tgt < T.end;
     const uint64_t vmask = __ballot(valid);
@@ -906,7 +906,7 @@ __global__ __launch_bounds__(64 * K) void k_walk_oct_ordered_frames(WalkArgs a) 
 
     const int lane = lane_id(), wv = uniform_i32(threadIdx.x / kWave), bit = target_bit<true>();
     const int row = lane / kRowTargets;
-    const int64_t sub = xcd_block(blockIdx.x, gridDim.x);
+    const int64_t sub = walk_block<FOREST>();
     const WaveTask T = wave_task<FOREST>(a, sub / 4);
     const int64_t tgt = T.base + (sub % 4) * kRowTargets + bit;
     const bool valid = tgt < T.end;

@@ -540,7 +540,7 @@ template <bool OCT, bool QUAD, bool SOFT, int STATS, bool FOREST, int K>
 __device__ __forceinline__ void walk_fast(const WalkArgs &a, WaveLds<OCT, QUAD> *lds, double (*cls)[kClasses][3][kSub]) {
     const int lane = lane_id();
     const int wv = uniform_i32(threadIdx.x / kWave);
-    const int64_t gw = (int64_t)xcd_block(blockIdx.x, gridDim.x) * kFastWaves + wv;
+    const int64_t gw = (int64_t)walk_block<FOREST>() * kFastWaves + wv;
     const int64_t sub = gw / K;
     const int k = (int)(gw - sub * K);
     const WaveTask T = wave_task<FOREST>(a, sub / kRows);
