@@ -218,6 +218,7 @@ __global__ __launch_bounds__(kGroupThreads) void k_group_targets(const float4 *_
         split_segments<64>(v, cnt, s_pos, s_box, s_key);
         split_segments<32>(v, cnt, s_pos, s_box, s_key);
         uint32_t *const order = &s_key[0][0];
+        __syncthreads();  // a wave may still read what the last exchange across waves (512 slots) left in s_key
 #pragma unroll
         for (int e = 0; e < kSlots; ++e) order[t * kSlots + e] = v[e] & (kGroupBlock - 1);
         __syncthreads();

@@ -1,0 +1,60 @@
+"""Kernels run on the CPU, a workgroup's threads as fibres that go on until
+they need one another (tests/native/simt.hpp): a wave gets as far ahead of the
+others as the barriers let it, whatever the order of the waves, and
+AddressSanitizer sees every access.  For races and reads out of bounds, which
+no GPU run would show."""
+
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "n-body_amd", "csrc")
+NATIVE = os.path.join(ROOT, "tests", "native")
+
+
+def _clang():
+    for c in ("/opt/rocm/lib/llvm/bin/clang++", "/opt/rocm/llvm/bin/clang++", shutil.which("clang++")):
+        if c and os.path.exists(c):
+            return c
+    return None
+
+
+pytestmark = pytest.mark.skipif(_clang() is None, reason="needs clang++")
+
+
+def _build(out, check, kernels, asan):
+    """The check program with the kernel files it needs, built in parallel."""
+    flags = [_clang(), "-std=c++17", "-O1", "-g", "-w", "-ffp-contract=off", "-D__HIP_PLATFORM_AMD__",
+             "-I/opt/rocm/include", "-I" + CSRC]
+    if asan:
+        flags += ["-fsanitize=address", "-fno-omit-frame-pointer", "-DSIMT_REDZONES"]
+    jobs, objs = [], []
+    for src in [os.path.join(CSRC, k + ".hip") for k in kernels] + [os.path.join(NATIVE, f) for f in ("simt.cpp", check)]:
+        obj = os.path.join(out, os.path.basename(src) + ".o")
+        shim = ["-include", os.path.join(NATIVE, "simt.hpp")] if src.endswith(".hip") else []
+        jobs.append(subprocess.Popen([*flags, *shim, "-x", "c++", "-c", src, "-o", obj], stderr=subprocess.PIPE))
+        objs.append(obj)
+    for j in jobs:
+        err = j.communicate()[1]
+        assert j.returncode == 0, err.decode()[-4000:]
+    exe = os.path.join(out, "check")
+    subprocess.run([*flags, *objs, "-o", exe], check=True)
+    return exe
+
+
+def _run(exe, *args, order=0):
+    env = dict(os.environ, NBG_SIMT_ORDER=str(order), ASAN_OPTIONS="detect_leaks=0:detect_stack_use_after_return=0")
+    return subprocess.run([exe, *args], capture_output=True, text=True, timeout=600, env=env)
+
+
+def test_target_groups(tmp_path):
+    exe = _build(str(tmp_path), "targets_check.cpp", ["targets"], asan=False)
+    outs = []
+    for order in (0, 1, 2, 3):
+        r = _run(exe, order=order)
+        assert r.returncode == 0, f"order {order}\n" + r.stdout[-2000:] + r.stderr[-2000:]
+        outs.append(r.stdout)
+    assert len(set(outs)) == 1
