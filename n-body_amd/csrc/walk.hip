@@ -526,6 +526,10 @@ __global__ __launch_bounds__(64 * K) void k_walk_lbvh_ordered_frames(WalkArgs a)
     const bool valid = tgt < T.end;
     const uint64_t vmask = target_ballot<true>(valid);
     if (vmask == 0) return;  // the whole workgroup
+    if (FOREST && (T.root < 0 || T.root >= a.max_nodes)) {  // no root was found: the whole workgroup
+        if (threadIdx.x == 0) atomicOr(a.err, 2u);
+        return;
+    }
     const float4 me = valid ? a.targets[tgt] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     const NodeRec *__restrict__ nodes = a.nodes;
     const float4 *__restrict__ bodies = a.bodies;
@@ -912,6 +916,10 @@ __global__ __launch_bounds__(64 * K) void k_walk_oct_ordered_frames(WalkArgs a) 
     const bool valid = tgt < T.end;
     const uint64_t vmask = target_ballot<true>(valid);
     if (vmask == 0) return;  // the whole workgroup
+    if (FOREST && (T.root < 0 || T.root >= a.max_nodes)) {  // no root was found: the whole workgroup
+        if (threadIdx.x == 0) atomicOr(a.err, 2u);
+        return;
+    }
     const float4 me = valid ? a.targets[tgt] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     const OctRec *__restrict__ nodes = a.onodes;
     const float4 *__restrict__ bodies = a.bodies;

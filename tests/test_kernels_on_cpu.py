@@ -27,7 +27,7 @@ pytestmark = pytest.mark.skipif(_clang() is None, reason="needs clang++")
 
 def _build(out, check, kernels, asan):
     """The check program with the kernel files it needs, built in parallel."""
-    flags = [_clang(), "-std=c++17", "-O1", "-g", "-w", "-ffp-contract=off", "-D__HIP_PLATFORM_AMD__",
+    flags = [_clang(), "-std=c++17", "-O0", "-gline-tables-only", "-w", "-ffp-contract=off", "-D__HIP_PLATFORM_AMD__",
              "-I/opt/rocm/include", "-I" + CSRC]
     if asan:
         flags += ["-fsanitize=address", "-fno-omit-frame-pointer", "-DSIMT_REDZONES"]
@@ -58,3 +58,9 @@ def test_target_groups(tmp_path):
         assert r.returncode == 0, f"order {order}\n" + r.stdout[-2000:] + r.stderr[-2000:]
         outs.append(r.stdout)
     assert len(set(outs)) == 1
+
+
+def test_frames_without_a_root(tmp_path):
+    exe = _build(str(tmp_path), "frames_check.cpp", ["walk", "walk_fast"], asan=True)
+    r = _run(exe)
+    assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-4000:]
