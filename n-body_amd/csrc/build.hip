@@ -344,15 +344,21 @@ static void radix_passes(K *ka, uint32_t *va, K *kb, uint32_t *vb, int64_t n, in
     else radix_passes_i<K, 16>(ka, va, kb, vb, n, passes, shift, status, err, s);
 }
 
+// Low word of body v's key (an index out of range, which only a timed-out
+// look-back leaves, and which k_sort_runs reports, has none).
+__device__ __forceinline__ uint64_t low_word(const uint64_t *__restrict__ lo, uint32_t v, int64_t n) {
+    return (int64_t)v < n ? lo[v] : 0ull;
+}
+
 // Whether key b at position j precedes key a at position i of a run sorted by
 // prefix (both positions in the order of the original index).  lo: the low
 // words of two-word keys, by original index.
 template <typename K, bool LO>
 __device__ __forceinline__ bool precedes(K b, uint32_t bi, int64_t j, K a, uint64_t alo, int64_t i,
-                                         const uint64_t *__restrict__ lo) {
+                                         const uint64_t *__restrict__ lo, int64_t n) {
     if (b != a) return b < a;
     if (LO) {
-        const uint64_t bl = lo[bi];
+        const uint64_t bl = low_word(lo, bi, n);
         if (bl != alo) return bl < alo;
     }
     return j < i;
@@ -418,7 +424,7 @@ __global__ __launch_bounds__(256) void k_sort_runs(const K *__restrict__ kin, co
             return;
         }
         pos = b;
-        for (int64_t j = b; j < e; ++j) pos += precedes<K, LO>(kin[j], vin[j], j, a, alo, i, lo) ? 1 : 0;
+        for (int64_t j = b; j < e; ++j) pos += precedes<K, LO>(kin[j], vin[j], j, a, alo, i, lo, n) ? 1 : 0;
     }
     kout[pos] = a;
     vout[pos] = v;
@@ -447,7 +453,7 @@ __global__ __launch_bounds__(1024) void k_sort_long(K *__restrict__ kin, uint32_
         bool bad = false;
         for (int64_t i = tid; i + 1 < m; i += 1024) {
             const K k0 = kin[b + i], k1 = kin[b + i + 1];
-            if (k0 > k1 || (LO && k0 == k1 && lo[vin[b + i]] > lo[vin[b + i + 1]])) bad = true;
+            if (k0 > k1 || (LO && k0 == k1 && low_word(lo, vin[b + i], n) > low_word(lo, vin[b + i + 1], n))) bad = true;
         }
         if (bad) unsorted = 1;
         __syncthreads();
@@ -456,7 +462,7 @@ __global__ __launch_bounds__(1024) void k_sort_long(K *__restrict__ kin, uint32_
         const int plo = LO ? 5 : 0, passes = unsorted ? plo + (shift + 7) / 8 : 0;
         for (int p = 0; p < passes; ++p) {
             auto digit = [&](K k, uint32_t v) {
-                return p < plo ? (uint32_t)(lo[v] >> (8 * p)) & 0xFFu : (uint32_t)(k >> (8 * (p - plo))) & 0xFFu;
+                return p < plo ? (uint32_t)(low_word(lo, v, n) >> (8 * p)) & 0xFFu : (uint32_t)(k >> (8 * (p - plo))) & 0xFFu;
             };
             if (tid < kRadix) cnt[tid] = 0;
             __syncthreads();
@@ -507,7 +513,7 @@ __global__ __launch_bounds__(1024) void k_sort_long(K *__restrict__ kin, uint32_
             for (int64_t i = tid; i < m; i += 1024) { kout[b + i] = ka[i]; vout[b + i] = va[i]; }
         __syncthreads();
         if (LO)
-            for (int64_t i = tid; i < m; i += 1024) lo_out[b + i] = lo[vout[b + i]];
+            for (int64_t i = tid; i < m; i += 1024) lo_out[b + i] = low_word(lo, vout[b + i], n);
         __syncthreads();
         (void)lane;
     };

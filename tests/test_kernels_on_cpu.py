@@ -64,3 +64,9 @@ def test_frames_without_a_root(tmp_path):
     exe = _build(str(tmp_path), "frames_check.cpp", ["walk", "walk_fast"], asan=True)
     r = _run(exe)
     assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-4000:]
+
+
+def test_runs_after_a_failed_pass(tmp_path):
+    exe = _build(str(tmp_path), "sort_check.cpp", ["build"], asan=True)
+    r = _run(exe, "failed")
+    assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-4000:]
