@@ -8,6 +8,7 @@ import os
 import shutil
 import subprocess
 
+import numpy as np
 import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -70,3 +71,26 @@ def test_runs_after_a_failed_pass(tmp_path):
     exe = _build(str(tmp_path), "sort_check.cpp", ["build"], asan=True)
     r = _run(exe, "failed")
     assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-4000:]
+
+
+# n, leaf, max_depth, coincident bodies
+@pytest.mark.parametrize("n,leaf,depth,same", [(3000, 2, 12, 129), (700, 1, 32, 65), (1500, 64, 5, 700)])
+def test_octree_pass_in_bounds(octree_exe, tmp_path, nbg, orc, n, leaf, depth, same):
+    """Box to ORDERED walk with buffers exactly as large as the library makes
+    them: no access outside them, and the oracle's bits."""
+    b = nbg.plummer(n, seed=300 + n)
+    for a in (b.x, b.y, b.z):
+        a[n // 3:n // 3 + same] = a[n // 3]
+    np.concatenate([b.x, b.y, b.z, b.m]).tofile(tmp_path / "in")
+    r = _run(octree_exe, str(tmp_path / "in"), str(n), str(leaf), str(depth), "0.9", "1e-4", str(tmp_path / "out"), "0",
+             str(n))
+    assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-4000:]
+    acc = np.fromfile(tmp_path / "out", np.float32).reshape(n, 3)
+    t = orc.Tree(0, b.x, b.y, b.z, b.m, theta=0.9, leaf=leaf, max_depth=depth, eps2=1e-4)
+    assert np.array_equal(acc.view(np.uint32), np.asarray(t.accel(b.x, b.y, b.z)).view(np.uint32))
+
+
+@pytest.fixture(scope="module")
+def octree_exe(tmp_path_factory):
+    return _build(str(tmp_path_factory.mktemp("octree")), "octree_check.cpp", ["build", "octree", "walk", "walk_fast"],
+                  asan=True)
