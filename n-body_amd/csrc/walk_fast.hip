@@ -61,7 +61,8 @@ constexpr int kFlushEvery = 8;            // lists of 64 between additions to FP
 constexpr int kListCap = 3 * kWave;
 constexpr int kMaskCap = 2 * kWave;       // entries of a list with masks
 constexpr int kMixCap = 2 * kWave;
-constexpr int kLeafCap = kWave + kRows;   // leaves are expanded as soon as kRows wait; one step adds at most 64
+constexpr int kLeafKeep = 15;              // leaves are expanded while more wait
+constexpr int kLeafCap = kWave + kLeafKeep;  // leaves of one step: at most 64
 constexpr uint32_t kMaxFastIters = 1u << 28;
 
 // The stack holds sibling groups (first child, mask).  Steps pop up to 64
@@ -73,7 +74,7 @@ constexpr uint32_t kMaxFastIters = 1u << 28;
 // 136 and 206) as far as the LDS of four workgroups a CU holds it, three for
 // the quadrupoles: with 128 groups the linear BVH's steps degenerate to one
 // group and its walk of 1,048,576 bodies took 24.8 ms.
-constexpr int wide_groups(bool oct, bool quad) { return oct ? (quad ? 192 : 256) : (quad ? 400 : 512); }
+constexpr int wide_groups(bool oct, bool quad) { return oct ? (quad ? 176 : 256) : (quad ? 392 : 512); }
 constexpr int stack_groups(bool oct, bool quad) {
     return wide_groups(oct, quad) + kWave + (oct ? 8 * (kOctLevels + 2) : 72);  // a linear BVH has at most 64 levels
 }
@@ -91,6 +92,7 @@ struct WaveLds {
     uint16_t lq_mask[kLeafCap];
     uint16_t smask[kMaskCap];                // masks of src[end - 1 - e]
     uint16_t qmask[QUAD ? kMaskCap : 1];
+    uint32_t starts[2];                      // lanes at which a leaf's bodies start
 };
 
 // Orders this wave's LDS writes and reads among its lanes (the hardware keeps
@@ -105,6 +107,20 @@ __device__ __forceinline__ int rank_in(uint64_t b) {
 }
 
 __device__ __forceinline__ bool in_lane(uint64_t b) { return __builtin_amdgcn_inverse_ballot_w64(b); }
+
+__device__ __forceinline__ uint64_t lanes_below(int n) { return n >= kWave ? ~0ull : (1ull << n) - 1ull; }
+
+// Inclusive scan over the wave, in the vector unit (row shifts, then the rows'
+// last lanes broadcast to the rows after them).
+__device__ __forceinline__ int incl_scan(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);   // row_shr:1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15 to rows 1 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31 to rows 2 and 3
+    return v;
+}
 
 // 2 v + (this lane's bit of b), in one instruction.
 __device__ __forceinline__ uint32_t shift_in(uint32_t v, uint64_t b) {
@@ -370,11 +386,23 @@ struct FastWalk {
         lq += nl;
     }
 
-    // Bodies of the last queued leaves: up to four leaves of at most 16
-    // bodies, one per row, or one larger leaf 64 bodies at a time.
-    __device__ __forceinline__ void expand_leaves() {
+    // The next 64 bodies of the queued leaves, from the last one on, one a lane:
+    // a scan of the leaves' counts tells each lane its leaf, so that the lanes
+    // are full whatever the leaves hold.  A pass over 1,024 systems of 256 to
+    // 65,536 bodies, ms, at leaf size 16 / 32 / 64: linear BVH 38.7 / 53.2 /
+    // 73.1, octree 24.5 / 26.4 / 33.3; four leaves of at most 16 bodies or one
+    // larger leaf at a time took 40.9 / 87.0 / 94.7 and 26.5 / 34.3 / 43.6.
+    // Leaves of 20 bodies or more summed by themselves, without the list and
+    // its masks: 10 to 20 % slower (part-filled chunks cost more than masks).
+    struct Bodies {
+        float4 b;    // a lane's body
+        uint32_t m;  // the targets that take it
+        int n;       // lanes with a body
+    };
+    __device__ __forceinline__ Bodies next_bodies() {
         lds_order();
-        const int e = lq - 1 - row;
+        // lane = queued leaf
+        const int e = lq - 1 - lane;
         int first = 0, cnt = 0;
         uint32_t m = 0;
         if (e >= 0) {
@@ -382,23 +410,44 @@ struct FastWalk {
             cnt = L.lq_cnt[e];
             m = L.lq_mask[e];
         }
-        if (__ballot(cnt > kSub) == 0) {
-            const int j = lane & (kSub - 1);
-            list_source(__ballot(j < cnt), a.bodies[j < cnt ? first + j : 0], m);
-            lq -= lq < kRows ? lq : kRows;
-            sum_ready();
-            return;
+        // a leaf's bodies go to the lanes from excl on
+        const int c = cnt < kWave + 1 ? cnt : kWave + 1;
+        const int incl = incl_scan(c), excl = incl - c;
+        if (lane < 2) L.starts[lane] = 0;
+        lds_order();
+        if (c > 0 && excl < kWave) atomicOr(&L.starts[excl >> 5], 1u << (excl & 31));
+        const int done = __popcll(__ballot(e >= 0 && incl <= kWave));
+        if (e >= 0 && excl < kWave && incl > kWave) {  // the rest of this leaf waits
+            L.lq_first[e] = first + (kWave - excl);
+            L.lq_cnt[e] = cnt - (kWave - excl);
         }
-        // row 0 holds the last entry
-        first = uniform_i32(first);
-        cnt = uniform_i32(cnt);
-        m = (uint32_t)uniform_i32((int)m);
-        lq -= 1;
-        for (int j0 = 0; j0 < cnt; j0 += kWave) {
-            const int j = j0 + lane;
-            list_source(__ballot(j < cnt), a.bodies[j < cnt ? first + j : 0], m);
-            sum_ready();
+        lq -= done;
+        lds_order();
+        const uint64_t starts = uniform_u64((uint64_t)L.starts[1] << 32 | L.starts[0]);
+        const int from = 4 * rank_in(starts >> 1);  // lane of this lane's leaf, in bytes
+        const int at = __builtin_amdgcn_ds_bpermute(from, first - excl) + lane;
+        Bodies r;
+        r.m = (uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)m);
+        const int total = __builtin_amdgcn_readlane(incl, kWave - 1);
+        r.n = total < kWave ? total : kWave;
+        r.b = a.bodies[lane < r.n ? at : 0];
+        return r;
+    }
+    __device__ __forceinline__ void list_bodies(const Bodies &v) {
+        list_source(lanes_below(v.n), v.b, v.m);
+        sum_ready();
+    }
+    // Lists bodies of the queued leaves while more than `keep` leaves wait; the
+    // next ones are on their way while the present ones are listed and summed.
+    __device__ __forceinline__ void expand_leaves(int keep) {
+        if (lq <= keep) return;
+        Bodies now = next_bodies();
+        while (lq > keep) {
+            const Bodies then = next_bodies();
+            list_bodies(now);
+            now = then;
         }
+        list_bodies(now);
     }
 
     // The criterion against the targets' box: the lanes whose node every point
@@ -526,10 +575,9 @@ struct FastWalk {
             else step();
             if (__ballot(fail)) break;
             sum_ready();
-            while (lq >= kRows) expand_leaves();
+            expand_leaves(sp > 0 || mq > 0 ? kLeafKeep : 0);
         }
         if (__ballot(fail)) return;  // the lists may hold more than a walk that went on would leave in them
-        while (lq > 0) expand_leaves();
         sum_rest();
     }
 };

@@ -1,6 +1,6 @@
-// A whole ORDERED octree pass on the CPU, every buffer exactly as large as the
+// A whole octree pass on the CPU, every buffer exactly as large as the
 // library makes it: box, keys, sort, topology, gather, summaries and the walk.
-//   octree_check FILE N LEAF DEPTH THETA EPS2 OUT FROM TO
+//   octree_check FILE N LEAF DEPTH THETA EPS2 OUT FROM TO ORDERED
 // FILE: x, y, z, m (N floats each); OUT: the accelerations of the walk's
 // targets FROM .. TO - 1 by body (others 0), and the interaction counts.
 #include <cstdio>
@@ -18,7 +18,7 @@ static void alloc(T **p, int64_t n) {
 }
 
 int main(int argc, char **argv) {
-    if (argc != 10) return 2;
+    if (argc != 11) return 2;
     const int64_t n = std::atoll(argv[2]), from = std::atoll(argv[8]), to = std::atoll(argv[9]);
     const int leaf = std::atoi(argv[3]), depth = std::atoi(argv[4]);
     const float theta = (float)std::atof(argv[5]), eps2 = (float)std::atof(argv[6]);
@@ -91,8 +91,9 @@ int main(int argc, char **argv) {
     w.ax = a[0]; w.ay = a[1]; w.az = a[2];
     w.counts = counts;
     w.err = &err;
-    w.split = ordered_split_waves((n + 63) / 64, true);
-    launch_walk_oct(w, 1, 1, nullptr);
+    const int ordered = std::atoi(argv[10]);
+    w.split = ordered ? ordered_split_waves((n + 63) / 64, true) : fast_split_waves((n + 63) / 64);
+    launch_walk_oct(w, ordered, 1, nullptr);
     std::printf("err %u pp %llu np %llu\n", err, counts[0], counts[1]);
     f = std::fopen(argv[7], "wb");
     std::vector<float> out(3 * n, 0.0f);

@@ -156,6 +156,20 @@ inline int __builtin_amdgcn_mov_dpp(int v, int ctrl, int, int, bool, SIMT_AT) {
     if (ctrl == 0x141) return simt_from<int>(w, (l & ~7) + (7 - (l & 7)));
     std::abort();
 }
+// row_shr (0x111 ..), row_bcast:15 and :31; lanes without a source take 0
+// (bound) or old, rows not in the mask old
+inline int __builtin_amdgcn_update_dpp(int old, int v, int ctrl, int rows, int, bool bound, SIMT_AT) {
+    uint64_t live;
+    const uint64_t *w = simt::meet(simt_word(v), &live, file, line);
+    const int l = simt::cur->lane;
+    if (!(rows >> (l / 16) & 1)) return old;
+    int from = -1;
+    if (ctrl > 0x110 && ctrl < 0x120) from = (l & 15) >= (ctrl & 15) ? l - (ctrl & 15) : -1;
+    else if (ctrl == 0x142) from = l >= 16 ? (l & ~15) - 1 : -1;
+    else if (ctrl == 0x143) from = l >= 32 ? 31 : -1;
+    else std::abort();
+    return from >= 0 ? simt_from<int>(w, from) : bound ? 0 : old;
+}
 inline bool __builtin_amdgcn_inverse_ballot_w64(uint64_t b) { return b >> simt::cur->lane & 1; }
 inline uint32_t __builtin_amdgcn_mbcnt_lo(uint32_t m, uint32_t a) {
     const int l = simt::cur->lane;

@@ -65,3 +65,45 @@ def test_full_stack(nbg, orc, gpu_ctx, solver, n, theta):
     assert s.counts() == (int(pp.sum()), int(npc.sum()))
     s.close()
     _check(got, want)
+
+
+@pytest.mark.parametrize("solver", list(SOLVERS))
+@pytest.mark.parametrize("leaf", [7, 31, 32, 63, 64, 65, 129])
+def test_leaves_fill_lanes(nbg, orc, gpu_ctx, solver, leaf):
+    """Leaves whose bodies end before, at and behind a wave's lanes, from leaves
+    of one body to one of more than all the queue holds."""
+    print(f"[walk] leaves {solver} leaf={leaf}", flush=True)
+    n = 4097
+    b = nbg.plummer(n, seed=leaf)
+    for v in (b.x, b.y, b.z):
+        v[:700] = v[0]
+    s = nbg.System(gpu_ctx, _params(nbg, solver, 0.6, leaf, 1e-4), n)
+    s.set_state(b)
+    acc = s.update_accelerations()
+    t = orc.Tree(SOLVERS[solver], b.x, b.y, b.z, b.m, theta=0.6, leaf=leaf, bits=63, eps2=1e-4)
+    want, pp, npc = t.accel(b.x, b.y, b.z, counts=True)
+    assert s.counts() == (int(pp.sum()), int(npc.sum()))
+    _check(acc, want)
+    s.close()
+
+
+@pytest.mark.parametrize("solver", ["lbvh", "octree"])
+def test_larger_leaves_cost_no_more_a_pair(nbg, gpu_ctx, solver):
+    """An interaction of a forest's pass takes less time at leaf size 32 than at
+    16, both with full lanes: 0.8 of it in both trees (with one leaf at a time,
+    1.09 in the linear BVH and 0.95 in the octree)."""
+    sizes = [6000 + 97 * k for k in range(96)]
+    per = {}
+    for leaf in (16, 32):
+        batch = nbg.Batch(gpu_ctx, sum(sizes), len(sizes), sum_mode=nbg.SUM_FAST)
+        for k, n in enumerate(sizes):
+            p = _params(nbg, solver, 0.5, leaf, 1e-4)
+            p.morton_bits = 30
+            batch.add(p, nbg.plummer(n, seed=k))
+        batch.update_accelerations()
+        pairs = sum(batch.counts())
+        ms = batch.autotune(leaf_sizes=(leaf,), repeats=10)[1][leaf]
+        batch.close()
+        per[leaf] = ms / pairs
+    print(f"[walk] {solver} ns a pair: {per[16] * 1e6:.4f} at leaf 16, {per[32] * 1e6:.4f} at 32", flush=True)
+    assert per[32] <= 0.9 * per[16]

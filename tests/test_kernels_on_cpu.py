@@ -83,11 +83,27 @@ def test_octree_pass_in_bounds(octree_exe, tmp_path, nbg, orc, n, leaf, depth, s
         a[n // 3:n // 3 + same] = a[n // 3]
     np.concatenate([b.x, b.y, b.z, b.m]).tofile(tmp_path / "in")
     r = _run(octree_exe, str(tmp_path / "in"), str(n), str(leaf), str(depth), "0.9", "1e-4", str(tmp_path / "out"), "0",
-             str(n))
+             str(n), "1")
     assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-4000:]
     acc = np.fromfile(tmp_path / "out", np.float32).reshape(n, 3)
     t = orc.Tree(0, b.x, b.y, b.z, b.m, theta=0.9, leaf=leaf, max_depth=depth, eps2=1e-4)
     assert np.array_equal(acc.view(np.uint32), np.asarray(t.accel(b.x, b.y, b.z)).view(np.uint32))
+
+
+@pytest.mark.parametrize("n,leaf,same", [(700, 16, 65), (500, 130, 0)])
+def test_fast_walk_in_bounds(octree_exe, tmp_path, nbg, orc, n, leaf, same):
+    """The FAST walk's lists, queues and stack, the waves in a shuffled order:
+    no access out of bounds, and the oracle's interaction counts."""
+    b = nbg.plummer(n, seed=300 + n)
+    for a in (b.x, b.y, b.z):
+        a[n // 3:n // 3 + same] = a[n // 3]
+    np.concatenate([b.x, b.y, b.z, b.m]).tofile(tmp_path / "in")
+    r = _run(octree_exe, str(tmp_path / "in"), str(n), str(leaf), "20", "0.5", "1e-4", str(tmp_path / "out"), "0", str(n),
+             "0", order=3)
+    assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-4000:]
+    t = orc.Tree(0, b.x, b.y, b.z, b.m, theta=0.5, leaf=leaf, max_depth=20, eps2=1e-4)
+    _, pp, npc = t.accel(b.x, b.y, b.z, counts=True)
+    assert f"pp {int(pp.sum())} np {int(npc.sum())}" in r.stdout
 
 
 @pytest.fixture(scope="module")
