@@ -183,7 +183,8 @@ void launch_morton(const float *x, const float *y, const float *z, int64_t n, co
 // last kernel moves every key to its place within the run of keys that share
 // those bits, by its rank in the run (runs of one: a copy); runs of more than
 // kRunMax keys (bodies much closer than the box suggests) are sorted by one
-// workgroup each.  Sort phase at 10,000 bodies 103 -> 30 us (63-bit keys),
+// workgroup each, up to run_one keys; past that all keys are sorted again by
+// the whole grid.  Sort phase at 10,000 bodies 103 -> 30 us (63-bit keys),
 // 170 -> 33 (octree paths, 102 bits), at 1,048,576 bodies 366 -> 122 (octree).
 constexpr int64_t kRunMax = 256;
 constexpr uint32_t kFlagAgg = 1u << 30;
@@ -205,40 +206,54 @@ __global__ __launch_bounds__(kSortBlock) void k_radix_hist(const K *__restrict__
     dc.store(ghist);
 }
 
-template <typename K, int ITEMS>
-__global__ __launch_bounds__(kSortBlock) void k_onesweep(const K *__restrict__ kin, const uint32_t *__restrict__ vin,
-                                                         K *__restrict__ kout, uint32_t *__restrict__ vout,
-                                                         int64_t n, int shift, const uint32_t *__restrict__ ghist,
-                                                         uint32_t *status, uint32_t *tile_counter, uint32_t *err) {
-    constexpr int W = kSortBlock / kWave, TILE = kSortBlock * ITEMS;
-    __shared__ uint32_t s_tile;
-    __shared__ uint32_t s_wh[W][kRadix];
-    __shared__ uint32_t s_local_off[kRadix];
-    __shared__ uint32_t s_gadj[kRadix];
-    __shared__ uint32_t s_tmp[W];
-    __shared__ K s_k[TILE];
-    __shared__ uint32_t s_v[TILE];
+// The LDS of a tile of NT threads with ITEMS keys each.
+template <typename K, int NT, int ITEMS, bool SHARED>
+struct TileLds {
+    uint32_t wh[NT / kWave][kRadix];  // digit counts of the waves (cleared by the caller)
+    uint32_t local_off[kRadix], gadj[kRadix], tmp[NT / kWave];
+    K k[NT * ITEMS];
+    uint32_t v[NT * ITEMS];
+    uint8_t d[SHARED ? NT * ITEMS : 1];  // digits, where they come from the low words in memory
+};
 
+// Keys and payload that other workgroups write in the same kernel (SHARED) go
+// past this XCD's caches.
+template <bool SHARED, typename T>
+__device__ __forceinline__ T sort_load(const T *p) {
+    if constexpr (SHARED) return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else return *p;
+}
+template <bool SHARED, typename T>
+__device__ __forceinline__ void sort_store(T *p, T v) {
+    if constexpr (SHARED) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else *p = v;
+}
+
+// One tile of one pass: ghist holds the digits' counts over all keys, status
+// the pass's look-back words.
+template <typename K, int NT, int ITEMS, bool SHARED, typename Digit>
+__device__ __forceinline__ void radix_tile(TileLds<K, NT, ITEMS, SHARED> &S, const K *kin, const uint32_t *vin, K *kout,
+                                           uint32_t *vout, int64_t n, int64_t tile, const uint32_t *ghist,
+                                           uint32_t *status, uint32_t *err, Digit &&digit) {
+    constexpr int W = NT / kWave, TILE = NT * ITEMS;
     const int tid = threadIdx.x, lane = lane_id(), w = tid / kWave;
-    if (tid == 0) s_tile = atomicAdd(tile_counter, 1u);
-    for (int i = tid; i < W * kRadix; i += kSortBlock) (&s_wh[0][0])[i] = 0;
-    __syncthreads();
-    const int64_t tile = s_tile;
     const int64_t tile_base = tile * TILE;
     const int64_t wave_base = tile_base + (int64_t)w * (kWave * ITEMS);
 
     K key[ITEMS];
-    uint32_t val[ITEMS], rnk[ITEMS];
+    uint32_t val[ITEMS], rnk[ITEMS], dig[SHARED ? ITEMS : 1];
 #pragma unroll
     for (int j = 0; j < ITEMS; ++j) {
         const int64_t i = wave_base + j * kWave + lane;
-        if (i < n) { key[j] = kin[i]; val[j] = vin[i]; } else { key[j] = 0; val[j] = 0; }
+        if (i < n) { key[j] = sort_load<SHARED>(kin + i); val[j] = sort_load<SHARED>(vin + i); }
+        else { key[j] = 0; val[j] = 0; }
     }
     const uint64_t lt = lanemask_lt();
 #pragma unroll
     for (int j = 0; j < ITEMS; ++j) {
         const bool valid = (wave_base + j * kWave + lane) < n;
-        const uint32_t d = (uint32_t)(key[j] >> shift) & 0xFFu;
+        const uint32_t d = digit(key[j], val[j]);
+        if constexpr (SHARED) dig[j] = d;
         uint64_t peers = __ballot(valid);
 #pragma unroll
         for (int b = 0; b < 8; ++b) {
@@ -247,10 +262,10 @@ __global__ __launch_bounds__(kSortBlock) void k_onesweep(const K *__restrict__ k
             peers &= bit ? bb : ~bb;
         }
         uint32_t base = 0;
-        if (valid) base = s_wh[w][d];
+        if (valid) base = S.wh[w][d];
         const uint32_t below = __popcll(peers & lt);
         __builtin_amdgcn_wave_barrier();
-        if (valid && below == 0) s_wh[w][d] = base + __popcll(peers);
+        if (valid && below == 0) S.wh[w][d] = base + __popcll(peers);
         __builtin_amdgcn_wave_barrier();
         rnk[j] = base + below;
     }
@@ -258,64 +273,89 @@ __global__ __launch_bounds__(kSortBlock) void k_onesweep(const K *__restrict__ k
 
     // One thread per digit: exclusive prefix across waves, tile total.
     const uint32_t d = tid;
+    const bool has = NT == kRadix || tid < kRadix;
     uint32_t tot = 0;
+    if (has) {
 #pragma unroll
-    for (int ww = 0; ww < W; ++ww) {
-        uint32_t c = s_wh[ww][d];
-        s_wh[ww][d] = tot;
-        tot += c;
+        for (int ww = 0; ww < W; ++ww) {
+            uint32_t c = S.wh[ww][d];
+            S.wh[ww][d] = tot;
+            tot += c;
+        }
     }
     uint32_t *st = status + tile * kRadix;
-    st_relaxed_agent(st + d, (tile == 0 ? kFlagPrefix : kFlagAgg) | tot);
-    const uint32_t local_off = block_excl_scan<kSortBlock>(tot, s_tmp, nullptr);
-    const uint32_t gbase = block_excl_scan<kSortBlock>(ghist[d], s_tmp, nullptr);
+    if (has) st_relaxed_agent(st + d, (tile == 0 ? kFlagPrefix : kFlagAgg) | tot);
+    const uint32_t local_off = block_excl_scan<NT>(tot, S.tmp, nullptr);
+    const uint32_t gbase = block_excl_scan<NT>(has ? sort_load<SHARED>(ghist + d) : 0u, S.tmp, nullptr);
 
-    uint32_t excl = 0;
-    if (tile > 0) {
-        int64_t p = tile - 1;
-        uint32_t spins = 0;
-        while (p >= 0) {
-            const uint32_t sv = ld_acquire_agent(status + p * kRadix + d);
-            const uint32_t f = sv & kFlagMask;
-            if (f == 0) {
-                if (++spins > kSpinLimit) { atomicOr(err, 1u); break; }
-                __builtin_amdgcn_s_sleep(1);
-                continue;
+    if (has) {
+        uint32_t excl = 0;
+        if (tile > 0) {
+            int64_t p = tile - 1;
+            uint32_t spins = 0;
+            while (p >= 0) {
+                const uint32_t sv = ld_acquire_agent(status + p * kRadix + d);
+                const uint32_t f = sv & kFlagMask;
+                if (f == 0) {
+                    if (++spins > kSpinLimit) { atomicOr(err, 1u); break; }
+                    __builtin_amdgcn_s_sleep(1);
+                    continue;
+                }
+                excl += sv & kValueMask;
+                if (f == kFlagPrefix) break;
+                --p;
             }
-            excl += sv & kValueMask;
-            if (f == kFlagPrefix) break;
-            --p;
+            st_relaxed_agent(st + d, kFlagPrefix | (excl + tot));
         }
-        st_relaxed_agent(st + d, kFlagPrefix | (excl + tot));
+        S.local_off[d] = local_off;
+        S.gadj[d] = gbase + excl - local_off;
     }
-    s_local_off[d] = local_off;
-    s_gadj[d] = gbase + excl - local_off;
     __syncthreads();
 
 #pragma unroll
     for (int j = 0; j < ITEMS; ++j) {
         const bool valid = (wave_base + j * kWave + lane) < n;
         if (valid) {
-            const uint32_t dj = (uint32_t)(key[j] >> shift) & 0xFFu;
-            const uint32_t pos = s_local_off[dj] + s_wh[w][dj] + rnk[j];
-            s_k[pos] = key[j];
-            s_v[pos] = val[j];
+            uint32_t dj;
+            if constexpr (SHARED) dj = dig[j];
+            else dj = digit(key[j], val[j]);
+            const uint32_t pos = S.local_off[dj] + S.wh[w][dj] + rnk[j];
+            S.k[pos] = key[j];
+            S.v[pos] = val[j];
+            if constexpr (SHARED) S.d[pos] = (uint8_t)dj;
         }
     }
     __syncthreads();
     const int64_t rem = n - tile_base;
     const int ntile = rem < TILE ? (int)rem : TILE;
-    for (int i = tid; i < ntile; i += kSortBlock) {
-        const K k = s_k[i];
-        const uint32_t dj = (uint32_t)(k >> shift) & 0xFFu;
-        const uint32_t g = s_gadj[dj] + (uint32_t)i;
+    for (int i = tid; i < ntile; i += NT) {
+        const K k = S.k[i];
+        const uint32_t v = S.v[i];
+        uint32_t di;
+        if constexpr (SHARED) di = S.d[i];
+        else di = digit(k, v);
+        const uint32_t g = S.gadj[di] + (uint32_t)i;
         if ((int64_t)g < n) {  // always true unless a look-back timed out
-            kout[g] = k;
-            vout[g] = s_v[i];
+            sort_store<SHARED>(kout + g, k);
+            sort_store<SHARED>(vout + g, v);
         } else {
             atomicOr(err, 1u);
         }
     }
+}
+
+template <typename K, int ITEMS>
+__global__ __launch_bounds__(kSortBlock) void k_onesweep(const K *__restrict__ kin, const uint32_t *__restrict__ vin,
+                                                         K *__restrict__ kout, uint32_t *__restrict__ vout,
+                                                         int64_t n, int shift, const uint32_t *__restrict__ ghist,
+                                                         uint32_t *status, uint32_t *tile_counter, uint32_t *err) {
+    __shared__ TileLds<K, kSortBlock, ITEMS, false> S;
+    __shared__ uint32_t s_tile;
+    if (threadIdx.x == 0) s_tile = atomicAdd(tile_counter, 1u);
+    for (int i = threadIdx.x; i < kSortBlock / kWave * kRadix; i += kSortBlock) (&S.wh[0][0])[i] = 0;
+    __syncthreads();
+    radix_tile<K, kSortBlock, ITEMS, false>(S, kin, vin, kout, vout, n, s_tile, ghist, status, err,
+                                            [&](K k, uint32_t) { return (uint32_t)(k >> shift) & 0xFFu; });
 }
 
 // The radix passes over bits shift .. shift + 8 passes - 1 (status cleared,
@@ -325,7 +365,7 @@ static void radix_passes_i(K *ka, uint32_t *va, K *kb, uint32_t *vb, int64_t n, 
                            uint32_t *status, uint32_t *err, hipStream_t s) {
     const int64_t tiles = (n + kSortBlock * ITEMS - 1) / (kSortBlock * ITEMS);
     uint32_t *ghist = status;                       // passes * 256
-    uint32_t *counters = status + 8 * kRadix;       // passes
+    uint32_t *counters = status + 8 * kRadix;       // passes; from + 32 on: long runs, the longest
     uint32_t *tstat = status + kSortHeadWords;      // passes * tiles * 256
     for (int p = 0; p < passes; ++p) {
         hipLaunchKernelGGL((k_onesweep<K, ITEMS>), dim3((unsigned)tiles), dim3(kSortBlock), 0, s, ka, va, kb, vb, n,
@@ -377,11 +417,11 @@ __global__ __launch_bounds__(256) void k_sort_runs(const K *__restrict__ kin, co
     const K a = kin[i], pre = a >> shift;
     const uint32_t v = vin[i];
     if ((int64_t)v >= n) { atomicOr(err, 1u); return; }  // only after a timed-out look-back
-    const uint64_t alo = LO ? lo[v] : 0ull;
+    uint64_t alo = 0;
     int64_t pos = i;
     const bool left = i > 0 && (kin[i - 1] >> shift) == pre, right = i + 1 < n && (kin[i + 1] >> shift) == pre;
     if (left || right) {
-        // the run's ends, by galloping
+        // the run's ends, by galloping; of a long run, the end for its first key only
         int64_t b = i, e = i + 1;
         if (left) {
             int64_t out = -1;
@@ -389,6 +429,7 @@ __global__ __launch_bounds__(256) void k_sort_runs(const K *__restrict__ kin, co
                 const int64_t k = i - step;
                 if (k < 0) break;
                 if ((kin[k] >> shift) != pre) { out = k; break; }
+                if (step >= kRunMax) return;  // long
                 b = k;
             }
             while (b - out > 1) {
@@ -403,6 +444,7 @@ __global__ __launch_bounds__(256) void k_sort_runs(const K *__restrict__ kin, co
                 const int64_t k = i + step;
                 if (k >= n) break;
                 if ((kin[k] >> shift) != pre) { out = k; break; }
+                if (left && step >= kRunMax) return;
                 in = k;
             }
             while (out - in > 1) {
@@ -413,9 +455,9 @@ __global__ __launch_bounds__(256) void k_sort_runs(const K *__restrict__ kin, co
             e = out;
         }
         if (e - b > kRunMax) {
-            uint32_t slot = kSortLongRuns;
             if (i == b) {
-                slot = atomicAdd(nlong, 1u);
+                const uint32_t slot = atomicAdd(nlong, 1u);
+                atomicMax(nlong + 1, (uint32_t)(e - b));
                 if (slot < kSortLongRuns) {
                     longs[2 * slot] = (uint32_t)b;
                     longs[2 * slot + 1] = (uint32_t)(e - b);
@@ -424,27 +466,158 @@ __global__ __launch_bounds__(256) void k_sort_runs(const K *__restrict__ kin, co
             return;
         }
         pos = b;
+        if (LO) alo = lo[v];
         for (int64_t j = b; j < e; ++j) pos += precedes<K, LO>(kin[j], vin[j], j, a, alo, i, lo, n) ? 1 : 0;
     }
     kout[pos] = a;
     vout[pos] = v;
-    if (LO) lo_out[pos] = alo;
+    if (LO) lo_out[pos] = left || right ? alo : lo[v];
+}
+
+// Every key again, by the whole key, in one kernel: where a run is long, most
+// keys share the bits that the passes sorted by, and one workgroup's time with
+// it would grow with the run.  Sort phase, ms, of 1,000,000 bodies of which two
+// are 1,000 / 10,000 radii out, a workgroup a run and so: linear BVH 0.90 /
+// 2.80 -> 0.50 / 0.47, octree 2.65 / 4.06 -> 0.78 / 0.73.  The digit counts,
+// the radix passes (but for digits that all keys share) and the copy to the
+// output are stages of `tiles` tasks each, handed out by one counter in that
+// order; a stage takes some 40 us at that size, of which the look-back and
+// the fences are most.  A task waits for the stage before it, whose tasks
+// were all handed out earlier, to workgroups that run: no workgroup waits for
+// one that has not started, however few are on the GPU at a time.
+constexpr int kAllItems = 4, kAllTile = 1024 * kAllItems;
+template <typename K>
+using AllLds = TileLds<K, 1024, kAllItems, true>;
+
+template <typename K, bool LO>
+__device__ void sort_all(AllLds<K> &S, K *ka, uint32_t *va, K *kb, uint32_t *vb, int64_t n,
+                         const uint64_t *__restrict__ lo, uint64_t *__restrict__ lo_out, uint32_t *words,
+                         uint32_t *tstat, uint32_t *err) {
+    __shared__ uint32_t s_task, s_late, s_equal;  // s_equal: passes whose digit all keys share
+    constexpr int kLowPasses = LO ? 5 : 0, kPasses = kLowPasses + (int)sizeof(K);
+    static_assert(kPasses <= kSortAllPasses, "words for the counts");
+    uint32_t *ghist = words, *next = words + kSortAllPasses * kRadix, *done = next + 1;
+    const int tid = threadIdx.x;
+    const uint32_t tiles = (uint32_t)((n + kAllTile - 1) / kAllTile);
+    // the look-back words of three passes in turn: the next pass's are cleared
+    // while those of the pass before are no longer read
+    auto status_of = [&](int pass) { return tstat + (int64_t)(pass % 3) * tiles * kRadix; };
+    if (tid == 0) s_equal = 0;
+    bool counted = false;
+    int passes = kPasses;
+    for (;;) {
+        __syncthreads();
+        if (tid == 0) s_task = atomicAdd(next, 1u);
+        __syncthreads();
+        const uint32_t stage = s_task / tiles, tile = s_task % tiles;
+        if (stage > (uint32_t)passes + 1) return;
+        auto wait_for = [&](uint32_t before) {  // false: given up
+            if (tid == 0) {
+                uint32_t spins = 0;
+                s_late = 0;
+                while (ld_acquire_agent(done + before) < tiles) {
+                    if (++spins > kSpinLimit) { atomicOr(err, 1u); s_late = 1; break; }
+                    __builtin_amdgcn_s_sleep(8);
+                }
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");  // for the workgroup, with the barriers around it
+            }
+            __syncthreads();
+            return s_late == 0;
+        };
+        if (stage > 0 && !counted) {
+            if (!wait_for(0)) return;
+            for (int i = tid; i < kPasses * kRadix; i += 1024)
+                if (sort_load<true>(ghist + i) == (uint32_t)n) atomicOr(&s_equal, 1u << (i / kRadix));
+            __syncthreads();
+            counted = true;
+            passes = kPasses - __popc(s_equal);
+            if (stage > (uint32_t)passes + 1) return;
+        }
+        if (stage > 1 && !wait_for(stage - 1)) return;
+        const int64_t base = (int64_t)tile * kAllTile, end = base + kAllTile < n ? base + kAllTile : n;
+        auto digit = [&](int pass, K k, uint32_t v) {
+            return pass < kLowPasses ? (uint32_t)(low_word(lo, v, n) >> (8 * pass)) & 0xFFu
+                                     : (uint32_t)(k >> (8 * (pass - kLowPasses))) & 0xFFu;
+        };
+        if (stage <= (uint32_t)passes && tid < kRadix) st_relaxed_agent(status_of(stage) + tile * kRadix + tid, 0u);
+        if (stage == 0) {
+            uint32_t *h = reinterpret_cast<uint32_t *>(S.k);
+            static_assert(sizeof S.k >= kPasses * kRadix * 4, "the counts' place");
+            for (int i = tid; i < kPasses * kRadix; i += 1024) h[i] = 0;
+            __syncthreads();
+            for (int64_t i0 = base; i0 < end; i0 += 1024) {
+                const int64_t i = i0 + tid;
+                const bool ok = i < end;
+                const K k = ok ? ka[i] : K(0);
+                const uint32_t v = ok ? va[i] : 0u;
+                const uint64_t low = LO && ok ? low_word(lo, v, n) : 0ull;
+                const uint64_t in = __ballot(ok);
+                for (int p = 0; p < kPasses; ++p) {
+                    const uint32_t d = p < kLowPasses ? (uint32_t)(low >> (8 * p)) & 0xFFu
+                                                      : (uint32_t)(k >> (8 * (p - kLowPasses))) & 0xFFu;
+                    // most waves' keys share most digits: one addition for them all
+                    const uint32_t first = (uint32_t)uniform_i32((int)d);
+                    const bool same = __ballot(ok && d == first) == in;
+                    if (same ? lane_id() == 0 && in : ok) atomicAdd(&h[p * kRadix + d], same ? (uint32_t)__popcll(in) : 1u);
+                }
+            }
+            __syncthreads();
+            for (int i = tid; i < kPasses * kRadix; i += 1024)
+                if (h[i]) atomicAdd(&ghist[i], h[i]);
+        } else if (stage <= (uint32_t)passes) {
+            const int step = (int)stage - 1;
+            uint32_t todo = ((1u << kPasses) - 1u) & ~s_equal;
+            for (int k = 0; k < step; ++k) todo &= todo - 1;
+            const int p = __builtin_ctz(todo);
+            for (int i = tid; i < 1024 / kWave * kRadix; i += 1024) (&S.wh[0][0])[i] = 0;
+            __syncthreads();
+            const bool back = step & 1;
+            radix_tile<K, 1024, kAllItems, true>(S, back ? kb : ka, back ? vb : va, back ? ka : kb, back ? va : vb, n,
+                                                 tile, ghist + p * kRadix, status_of(step), err,
+                                                 [&](K k, uint32_t v) { return digit(p, k, v); });
+        } else {
+            for (int64_t i = base + tid; i < end; i += 1024) {
+                const uint32_t v = sort_load<true>((passes & 1 ? vb : va) + i);
+                if (!(passes & 1)) {
+                    kb[i] = sort_load<true>(ka + i);
+                    vb[i] = v;
+                }
+                if (LO) lo_out[i] = low_word(lo, v, n);
+            }
+        }
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's stores have arrived
+        __syncthreads();
+        if (tid == 0) {
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+            atomicAdd(done + stage, 1u);
+        }
+    }
 }
 
 // The runs that k_sort_runs left: one workgroup sorts one run at a time by its
 // low digits (LSD, stable), the run's two buffers in turn.  More long runs
-// than the list holds: every workgroup looks for the runs' heads itself.
+// than the list holds: every workgroup looks for the runs' heads itself.  A
+// run of more than run_one keys: all keys are sorted again (sort_all, 100 to
+// 300 us below 100,000 keys; one workgroup takes 10 us for each 1,024 keys of
+// the longest run, 25 with low words).
+constexpr uint32_t run_one(bool lo) { return lo ? 4096 : 16384; }
 template <typename K, bool LO>
 __global__ __launch_bounds__(1024) void k_sort_long(K *__restrict__ kin, uint32_t *__restrict__ vin,
                                                     K *__restrict__ kout, uint32_t *__restrict__ vout, int64_t n,
                                                     int shift, const uint64_t *__restrict__ lo,
                                                     uint64_t *__restrict__ lo_out, const uint32_t *nlong,
-                                                    const uint32_t *longs) {
+                                                    const uint32_t *longs, uint32_t *words, uint32_t *tstat,
+                                                    uint32_t *err) {
     constexpr int W = 1024 / kWave;
     __shared__ uint32_t cnt[kRadix], wh[W][kRadix], tmp[W];
     __shared__ int unsorted;
-    const uint32_t runs = *nlong;
+    const uint32_t runs = nlong[0];
     if (runs == 0) return;
+    if (nlong[1] > run_one(LO)) {
+        __shared__ AllLds<K> S;
+        sort_all<K, LO>(S, kin, vin, kout, vout, n, lo, lo_out, words, tstat, err);
+        return;
+    }
     const int tid = threadIdx.x, lane = lane_id(), w = tid / kWave;
     auto sort_run = [&](int64_t b, int64_t m) {
         // already in order (coincident bodies): a copy
@@ -558,7 +731,7 @@ static void sort_planned(K *keys, uint32_t *idx, K *keys_alt, uint32_t *idx_alt,
     uint32_t *va = plan.from_alt ? idx_alt : idx, *vb = plan.from_alt ? idx : idx_alt;
     radix_passes(ka, va, kb, vb, n, plan.passes, plan.shift, status, err, s);
     if (!plan.runs) return;
-    uint32_t *nlong = status + 8 * kRadix + 32, *longs = status + 8 * kRadix + 64;
+    uint32_t *nlong = status + 8 * kRadix + 32, *longs = status + 8 * kRadix + 64, *words = longs + 2 * kSortLongRuns;
     const dim3 g((unsigned)((n + 255) / 256));
     const unsigned gl = n <= kRunMax ? 0u : (unsigned)(n / kRunMax < 256 ? n / kRunMax : 256);
     if (lo) {
@@ -566,13 +739,13 @@ static void sort_planned(K *keys, uint32_t *idx, K *keys_alt, uint32_t *idx_alt,
                            lo_sorted, nlong, longs, err);
         if (gl)
             hipLaunchKernelGGL((k_sort_long<K, true>), dim3(gl), dim3(1024), 0, s, keys_alt, idx_alt, keys, idx, n,
-                               plan.shift, lo, lo_sorted, nlong, longs);
+                               plan.shift, lo, lo_sorted, nlong, longs, words, status + kSortHeadWords, err);
     } else {
         hipLaunchKernelGGL((k_sort_runs<K, false>), g, dim3(256), 0, s, keys_alt, idx_alt, keys, idx, n, plan.shift, lo,
                            lo_sorted, nlong, longs, err);
         if (gl)
             hipLaunchKernelGGL((k_sort_long<K, false>), dim3(gl), dim3(1024), 0, s, keys_alt, idx_alt, keys, idx, n,
-                               plan.shift, lo, lo_sorted, nlong, longs);
+                               plan.shift, lo, lo_sorted, nlong, longs, words, status + kSortHeadWords, err);
     }
 }
 

@@ -30,9 +30,11 @@ constexpr int64_t sort_tiles_upto(int64_t n) {
 }
 constexpr int sort_passes(int key_bits) { return (key_bits + 7) / 8; }
 // Words of status memory one sort needs: histograms, tile counters, the list
-// of long runs, and per pass the tiles' look-back words.
-constexpr int kSortLongRuns = 4096;
-constexpr int64_t kSortHeadWords = 8 * kRadix + 64 + 2 * kSortLongRuns;
+// of long runs, what the sort of all keys after a long run counts in, and per
+// pass the tiles' look-back words (that sort uses three passes' of them, for
+// tiles that are no smaller).
+constexpr int kSortLongRuns = 4096, kSortAllPasses = 13;
+constexpr int64_t kSortHeadWords = 8 * kRadix + 64 + 2 * kSortLongRuns + (kSortAllPasses + 1) * kRadix;
 constexpr int64_t sort_status_words(int64_t n, int key_bits) {
     return kSortHeadWords + (int64_t)sort_passes(key_bits) * (sort_tiles_upto(n) * kRadix);
 }

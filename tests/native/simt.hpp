@@ -124,6 +124,7 @@ inline void __builtin_amdgcn_fence(int, const char *scope, SIMT_AT) {
     if (scope[0] == 'w' && scope[1] == 'a') simt::meet(0, &live, file, line);
 }
 inline void __builtin_amdgcn_s_sleep(int) {}
+inline void __builtin_amdgcn_s_waitcnt(int) {}
 inline int __builtin_amdgcn_ds_bpermute(int addr, int v, SIMT_AT) {
     uint64_t live;
     return simt_from<int>(simt::meet(simt_word(v), &live, file, line), addr / 4);
@@ -196,6 +197,11 @@ inline T simt_rmw_add(T *p, U v) {
 inline uint32_t atomicAdd(uint32_t *p, uint32_t v) { return simt_rmw_add(p, v); }
 inline int atomicAdd(int *p, int v) { return simt_rmw_add(p, v); }
 inline unsigned long long atomicAdd(unsigned long long *p, unsigned long long v) { return simt_rmw_add(p, v); }
+inline uint32_t atomicMax(uint32_t *p, uint32_t v) {
+    const uint32_t o = *p;
+    if (v > o) *p = v;
+    return o;
+}
 inline uint32_t atomicOr(uint32_t *p, uint32_t v) {
     const uint32_t o = *p;
     *p = o | v;

@@ -1,6 +1,9 @@
 // The last stage of the build's sort (build.hip) on the CPU.
 //   failed: indices as a radix pass leaves them that gave up its look-back
 //     (some never written): an error is reported, nothing is read out of bounds.
+//   runs: keys that share the sorted bits in runs on both sides of the run
+//     lengths at which the stage changes its way: the stable order.
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -38,9 +41,58 @@ static int failed() {
     return bad;
 }
 
+static int runs() {
+    int bad = 0;
+    // lengths of the runs, one after the other, until n keys are there
+    const std::vector<std::vector<int>> shapes = {{256, 257, 1, 3}, {4096, 1, 300}, {4097, 2}, {9000}, {300}, {5, 20000, 700}, {16384, 9}, {16385, 9}};
+    for (size_t q = 0; q < shapes.size(); ++q)
+        for (int lo = 0; lo < 2; ++lo) {
+            const int n = 12345 + 8191 * (int)(q % 3);
+            const SortPlan plan{0, 31, true, true};
+            std::vector<uint64_t> keys(n), alt(n), low(n), low_out(n);
+            std::vector<uint32_t> idx(n), idx_alt(n), status((size_t)sort_status_words(n, 64), 0xA5A5A5A5u);
+            std::fill(status.begin(), status.begin() + sort_clear_words(n, plan), 0u);
+            std::mt19937_64 g(q);
+            uint64_t prefix = 0;
+            for (int i = 0, r = 0; i < n; ++prefix, ++r)
+                for (int k = shapes[q][r % shapes[q].size()]; k > 0 && i < n; --k, ++i)
+                    alt[i] = prefix << 31 | (g() & (g() % 7 ? 0x7FFFFFFFull : 0x3ull));
+            // equal prefixes stand in the order of the index
+            std::vector<uint32_t> at(n);
+            for (int i = 0; i < n; ++i) at[i] = (uint32_t)i;
+            std::shuffle(at.begin(), at.end(), g);
+            for (int i = 0; i < n;) {
+                int e = i;
+                while (e < n && alt[e] >> 31 == alt[i] >> 31) ++e;
+                std::sort(at.begin() + i, at.begin() + e);
+                i = e;
+            }
+            for (int i = 0; i < n; ++i) {
+                idx_alt[i] = at[i];
+                low[at[i]] = lo ? g() & (g() % 3 ? 0x7FFFFFFFFFull : 0x7ull) : 0;
+            }
+            struct E { uint64_t k, l; uint32_t v; };
+            std::vector<E> want(n);
+            for (int i = 0; i < n; ++i) want[i] = E{alt[i], low[at[i]], at[i]};
+            std::sort(want.begin(), want.end(), [](const E &a, const E &b) {
+                return a.k != b.k ? a.k < b.k : a.l != b.l ? a.l < b.l : a.v < b.v;
+            });
+            uint32_t err = 0;
+            launch_sort(keys.data(), idx.data(), alt.data(), idx_alt.data(), n, 63, plan, status.data(), &err, nullptr,
+                        lo ? low.data() : nullptr, lo ? low_out.data() : nullptr);
+            int wrong = err != 0;
+            for (int i = 0; i < n; ++i)
+                wrong += keys[i] != want[i].k || idx[i] != want[i].v || (lo && low_out[i] != want[i].l);
+            std::printf("runs %zu lo=%d n=%d wrong %d\n", q, lo, n, wrong);
+            bad += wrong != 0;
+        }
+    return bad;
+}
+
 int main(int argc, char **argv) {
     int bad = 0;
     if (argc > 1 && !std::strcmp(argv[1], "failed")) bad = failed();
+    if (argc > 1 && !std::strcmp(argv[1], "runs")) bad = runs();
     if (bad) std::printf("%d wrong\n", bad);
     return bad != 0;
 }

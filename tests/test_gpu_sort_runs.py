@@ -21,6 +21,11 @@ def _bodies(nbg, kind, n):
         c = np.repeat(r.uniform(-1, 1, (3, n // 260 + 1)), 260, axis=1)[:, :n]
         p = (c + 1e-5 * r.uniform(-1, 1, (3, n))).astype(np.float32)
         p = p[:, r.permutation(n)]
+    elif kind == "escapers":  # two bodies ten thousand sides out
+        p = np.stack([b.x, b.y, b.z])
+        p[:, 0], p[:, -1] = -10000.0, 10000.0
+        b.x, b.y, b.z = (np.ascontiguousarray(v) for v in p)
+        return b
     else:
         return b
     p[:, :1], p[:, -1:] = -1.0, 1.0
@@ -37,7 +42,8 @@ def _params(nbg, solver, bits, leaf=16):
 
 @pytest.mark.parametrize("bits", [30, 63])
 @pytest.mark.parametrize("kind,n", [("cube", 1), ("cube", 2), ("cube", 1023), ("cube", 1025), ("cube", 262145),
-                                    ("cluster", 258), ("cluster", 5000), ("cluster", 40000), ("coincident", 3000),
+                                    ("cluster", 258), ("cluster", 5000), ("cluster", 40000), ("cluster", 16386), ("cluster", 16387),
+                                    ("cluster", 300001), ("escapers", 1200000), ("coincident", 3000), ("coincident", 70000),
                                     ("clusters", 5001), ("clusters", 90000), ("clusters", 1200000)])
 def test_linear_bvh_order(nbg, orc, gpu_ctx, kind, n, bits):
     print(f"[sort] {kind} n={n} bits={bits}", flush=True)
@@ -54,7 +60,8 @@ def test_linear_bvh_order(nbg, orc, gpu_ctx, kind, n, bits):
     assert np.array_equal(keys, want[order])
 
 
-@pytest.mark.parametrize("kind,n,leaf", [("cluster", 300, 1), ("cluster", 6000, 16), ("coincident", 700, 4),
+@pytest.mark.parametrize("kind,n,leaf", [("cluster", 300, 1), ("cluster", 6000, 16), ("cluster", 20000, 16),
+                                         ("escapers", 150000, 8), ("coincident", 700, 4),
                                          ("clusters", 9000, 8), ("cube", 257, 1)])
 def test_octree_bits(nbg, orc, gpu_ctx, kind, n, leaf):
     print(f"[sort] octree {kind} n={n} leaf={leaf}", flush=True)
@@ -69,3 +76,29 @@ def test_octree_bits(nbg, orc, gpu_ctx, kind, n, leaf):
     assert np.array_equal(acc.view(np.uint32), want.view(np.uint32))
     assert s.counts() == (int(pp.sum()), int(npc.sum()))
     s.close()
+
+
+@pytest.mark.parametrize("solver", ["LINEAR_BVH", "BARNES_HUT"])
+@pytest.mark.parametrize("n", [100000, 1000000])
+def test_escapers_cost(nbg, gpu_ctx, solver, n):
+    """Two bodies far out put all others into a few runs.  The sort then takes
+    twice the passes or three times: at 1,000,000 bodies 5 (linear BVH) and 7
+    (octree) times the plain sort.  One workgroup with such a run took 26 and
+    34 times."""
+    ms = {}
+    for kind in ("cube", "escapers"):
+        b = _bodies(nbg, kind, n)
+        p = _params(nbg, getattr(nbg, solver), 63)
+        p.theta = 1.0
+        s = nbg.System(gpu_ctx, p, n)
+        s.set_state(b)
+        s.enable_counts(False)
+        s.enable_timing(True)
+        times = []
+        for _ in range(5):
+            s.update_accelerations()
+            times.append(s.phase_times()["sort"])
+        ms[kind] = min(times)
+        s.close()
+    print(f"[sort] {solver} n={n} ms {ms}", flush=True)
+    assert ms["escapers"] <= 12 * ms["cube"]

@@ -67,9 +67,10 @@ def test_frames_without_a_root(tmp_path):
     assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-4000:]
 
 
-def test_runs_after_a_failed_pass(tmp_path):
+@pytest.mark.parametrize("what", ["failed", "runs"])
+def test_last_stage_of_the_sort(tmp_path, what):
     exe = _build(str(tmp_path), "sort_check.cpp", ["build"], asan=True)
-    r = _run(exe, "failed")
+    r = _run(exe, what)
     assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-4000:]
 
 
