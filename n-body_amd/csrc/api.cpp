@@ -152,7 +152,7 @@ int ensure_octree(nbg_sys *s) {
     A(&b.key_hi, n); A(&b.key_lo, n); A(&b.lo_sorted, n);
     A(&b.nown, n); A(&b.nbase, n);
     A(&b.nfirst, cap); A(&b.ncount, cap); A(&b.nparent, cap); A(&b.nmeta, cap);
-    A(&b.occ, cap); A(&b.cb, cap); A(&b.flags, cap); A(&b.glist, 2 * (cap + 64));
+    A(&b.occ, cap); A(&b.cb, cap); A(&b.flags, cap); A(&b.glist, 2 * oct_queue_words(n));
     A(&b.scan_ws, oct_scan_words(n, cap));
     A(&b.nodes, cap); A(&b.centre, cap); A(&b.thr, 64); A(&b.misc, 64);
     if (r != NBG_OK) {

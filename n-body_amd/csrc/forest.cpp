@@ -230,7 +230,7 @@ int ensure_octree(nbg_batch *b) {
         A(&o.key_hi, n); A(&o.key_lo, n); A(&o.lo_sorted, n); A(&o.nown, n); A(&o.nbase, n);
         A(&o.targets, n);
         A(&o.nfirst, cap); A(&o.ncount, cap); A(&o.nparent, cap); A(&o.nmeta, cap);
-        A(&o.occ, cap); A(&o.cb, cap); A(&o.flags, cap); A(&o.glist, 2 * (cap + 64));
+        A(&o.occ, cap); A(&o.cb, cap); A(&o.flags, cap); A(&o.glist, 2 * oct_queue_words(n));
         A(&o.scan_ws, oct_scan_words(n, cap));
         A(&o.nodes, cap); A(&o.centre, cap); A(&o.thr, (int64_t)kOctThrStride * b->cap_s); A(&o.misc, 64);
         if (r != NBG_OK) {

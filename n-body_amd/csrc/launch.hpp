@@ -151,7 +151,7 @@ struct OctBuffers {
     uint32_t *occ = nullptr;       // cap: occupied-child octant mask
     uint32_t *cb = nullptr;        // cap: child counts, then their exclusive scan
     uint32_t *flags = nullptr;     // cap: summary arrival counters
-    uint32_t *glist = nullptr;     // 2 * (cap + 64): two queues of straddling parents (summaries)
+    uint32_t *glist = nullptr;     // 2 * oct_queue_words(n): two queues of straddling parents (summaries)
     uint32_t *scan_ws = nullptr;   // the scan tiles' sums of nown, then of cb (oct_scan_words)
     OctRec *nodes = nullptr;       // cap, by slot
     float4 *centre = nullptr;      // cap, by slot: cell centre xyz, side
@@ -160,6 +160,9 @@ struct OctBuffers {
     uint32_t *sums_own() const { return scan_ws; }
     uint32_t *sums_child() const { return scan_ws + (n + kScanTile - 1) / kScanTile; }
 };
+// The summaries' queue: a place for each body, a count for each kOctSegment of them.
+constexpr int kOctSegment = 1024;
+inline int64_t oct_queue_words(int64_t n) { return n + (n + kOctSegment - 1) / kOctSegment; }
 inline int64_t oct_scan_words(int64_t n, int64_t cap) {
     return (n + kScanTile - 1) / kScanTile + (cap + kScanTile - 1) / kScanTile + 1;
 }
@@ -169,8 +172,6 @@ inline void oct_fills(FillSet &f, const OctBuffers &ob, int64_t n, int32_t *leaf
     f.add(ob.occ, ob.cap);
     f.add(leaf_start, n, 0xFFFFFFFFu);
     f.add(ob.flags, ob.cap);
-    f.add(ob.glist, 64);
-    f.add(ob.glist + ob.cap + 64, 64);
 }
 // What a linear-BVH build of n bodies counts in, to be set before it.
 inline void lbvh_fills(FillSet &f, int64_t n, int32_t *leaf_start, uint32_t *scan_ws, uint32_t *flags) {

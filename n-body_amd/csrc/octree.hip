@@ -444,13 +444,23 @@ __global__ __launch_bounds__(256) void k_oct_leafsort(int64_t n, const int32_t *
 // (Tree::summarizeTreeTop, Trees/Tree.h:196-216), giving 0/0 = NaN there and
 // so a NaN root COM whenever a level-1 octant is empty.
 //
-// Scheduling as for the LBVH: workgroups own kOctSummBodies consecutive bodies,
-// climb with workgroup-scope arrival counters while the parent's range stays
-// inside, and queue straddling parents for one final workgroup.
+// Scheduling as for the LBVH: workgroups own kOctSegment consecutive bodies
+// and climb with workgroup-scope arrival counters while the parent's range
+// stays inside.  A parent that leaves the range is queued in place of the
+// arrival, at the workgroup's own positions of the queue, with a count; the
+// next pass's workgroups own kOctSummJoin times the bodies and go on from
+// their own segments of it, the last one from all.  With one queue, which
+// each workgroup of the middle pass read whole for its own entries, that pass
+// took 2.65 ms for 48 million bodies, now 0.07.  Summaries, us, one queue /
+// segments: 10,000 bodies 26 / 28, 100,000 35 / 37, 1,000,000 133 / 112,
+// 16,777,216 1,465 / 1,160; quadrupoles, 100,000 90 / 94, 300,000 179 / 163,
+// 4,000,000 646 / 547.  Bound by the chain of arrivals up to a few million
+// bodies, then by the leaves' lanes (one of eight has a leaf).
 
-constexpr int kOctSummBodies = 1024;                // bodies per workgroup in the local pass, one per thread
-constexpr int kOctSummMid = kOctSummBodies * 64;    // bodies per workgroup in the middle pass
-constexpr unsigned kOctSummMidMinBlocks = 8;        // fewer middle workgroups: no middle pass
+constexpr int kOctSummJoin = 64;   // segments that a workgroup of a middle pass joins
+constexpr int kOctSummLast = 128;  // and the last one: a pass less for 65,536 to 131,072 bodies (100,000: 37 us to 45)
+constexpr int kOctSummThreads = 1024;
+static_assert(kOctSegment == kOctSummThreads, "the local pass: a thread for each body");
 
 __device__ __forceinline__ uint32_t arrive(uint32_t *flag) {
     return __hip_atomic_fetch_add(flag, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -540,25 +550,15 @@ __device__ __forceinline__ void oct_summ_inner(int p, const OctRec &r, OctRec *n
     if (quad) oct_quad_inner(p, r, nodes, quad, com);
 }
 
-// JOIN: the places of the queue of straddling parents are taken one for all of
-// a workgroup instead of one by one: summaries us, 1,000,000 bodies 188 -> 135,
-// 300,000 101 -> 87; with quadrupoles 292 -> 268, but 300,007 190 -> 210: the
-// waves that wait for the workgroup's end hold registers that its neighbours'
-// climbs could use.
-template <bool JOIN>
-__global__ __launch_bounds__(kOctSummBodies) void k_oct_summ_local(const float4 *__restrict__ bodies, int64_t n,
-                                                        OctRec *nodes, const int32_t *__restrict__ leaf_start,
-                                                        const uint32_t *__restrict__ misc, uint32_t *flags,
-                                                        uint32_t *glist, int64_t glist_cap, float4 *quad,
-                                                        uint32_t *err) {
-    __shared__ uint32_t s_n, s_base, s_queue[JOIN ? kOctSummBodies : 1];
-    const int64_t lo = (int64_t)blockIdx.x * kOctSummBodies, hi = lo + kOctSummBodies;
-    const int64_t T = misc[0], i = lo + threadIdx.x;
-    if (JOIN) {
-        if (threadIdx.x == 0) s_n = 0;
-        __syncthreads();
-    }
-    int queued = -1;  // the straddling parent that this thread's climb ends at
+__global__ __launch_bounds__(kOctSummThreads) void k_oct_summ_local(const float4 *__restrict__ bodies, int64_t n,
+                                                         OctRec *nodes, const int32_t *__restrict__ leaf_start,
+                                                         const uint32_t *__restrict__ misc, uint32_t *flags,
+                                                         uint32_t *qout, uint32_t *qout_n, float4 *quad, uint32_t *err) {
+    __shared__ uint32_t s_queued, s_done;
+    const int64_t lo = (int64_t)blockIdx.x * kOctSegment, hi = lo + kOctSegment, i = lo + threadIdx.x;
+    const int64_t T = misc[0];
+    if (threadIdx.x == 0) s_queued = s_done = 0;
+    __syncthreads();
     const int s = i < n ? leaf_start[i] : -1;
     int4 t = make_int4(-1, 0, 0, -1);
     if (s >= 0 && s < T) t = nodes[s].topo;
@@ -572,15 +572,8 @@ __global__ __launch_bounds__(kOctSummBodies) void k_oct_summ_local(const float4 
         if (parent >= s || hops > kOctLevels) { atomicOr(err, 4u); break; }
         const OctRec r = nodes[parent];
         const int4 tp = r.topo;
-        const bool local = tp.x >= lo && (int64_t)tp.x + tp.y <= hi;
-        if (!local) {
-            if (JOIN) {
-                queued = parent;
-            } else {
-                const uint32_t k = atomicAdd(&glist[0], 1u);
-                if (k < glist_cap) glist[64 + k] = (uint32_t)parent;
-                else atomicOr(err, 4u);
-            }
+        if (!(tp.x >= lo && (int64_t)tp.x + tp.y <= hi)) {
+            qout[lo + atomicAdd(&s_queued, 1u)] = (uint32_t)parent;  // one for a leaf at most
             break;
         }
         if (arrive(&flags[parent]) + 1u < (uint32_t)oct_nchild(r)) break;
@@ -588,42 +581,41 @@ __global__ __launch_bounds__(kOctSummBodies) void k_oct_summ_local(const float4 
         oct_summ_inner(parent, r, nodes, quad);
         parent = tp.w;
     }
-    if (!JOIN) return;
-    if (queued >= 0) s_queue[atomicAdd(&s_n, 1u)] = (uint32_t)queued;
-    __syncthreads();
-    const uint32_t count = s_n;
-    if (threadIdx.x == 0 && count) s_base = atomicAdd(&glist[0], count);
-    __syncthreads();
-    for (uint32_t k = threadIdx.x; k < count; k += kOctSummBodies) {
-        const int64_t at = (int64_t)s_base + k;
-        if (at < glist_cap) glist[64 + at] = s_queue[k];
-        else atomicOr(err, 4u);
-    }
+    // the last wave stores the count: a barrier would keep the registers of
+    // the waves that are done (quadrupoles of 300,007 bodies 10 % slower)
+    __builtin_amdgcn_wave_barrier();
+    if (lane_id() == 0 && arrive(&s_done) + 1u == blockDim.x / kWave) qout_n[blockIdx.x] = s_queued;
 }
 
-// Middle pass (as the linear BVH's): workgroup g owns kOctSummMid bodies
-// and the queued parents whose first body lies there, climbs while the node
-// stays inside, and forwards a parent that leaves the range in place of the
-// arrival.
-__global__ __launch_bounds__(1024) void k_oct_summ_mid(OctRec *nodes, const uint32_t *__restrict__ misc,
-                                                       uint32_t *flags, const uint32_t *gin, uint32_t *gout,
-                                                       int64_t qcap, float4 *quad, uint32_t *err) {
+// A later pass: workgroup g owns the `range` bodies from g * range and the
+// parents that the workgroups of the pass before, of `from` bodies each,
+// queued there (a parent that stays inside gets all its arrivals from it).
+// 2^lanes threads take a segment's parents: no scan of the counts stands
+// before the climbs.  qout null: the last pass.
+__global__ __launch_bounds__(kOctSummThreads) void k_oct_summ_queue(OctRec *nodes, const uint32_t *__restrict__ misc,
+                                                                    uint32_t *flags, int64_t n,
+                                                                    const uint32_t *__restrict__ qin,
+                                                                    const uint32_t *__restrict__ qin_n, int64_t from,
+                                                                    int64_t range, int lanes, uint32_t *qout,
+                                                                    uint32_t *qout_n, float4 *quad, uint32_t *err) {
+    __shared__ uint32_t s_queued;
     const int64_t T = misc[0];
-    const int64_t lo = (int64_t)blockIdx.x * kOctSummMid, hi = lo + kOctSummMid;
-    const uint32_t cnt = gin[0] < qcap ? gin[0] : (uint32_t)qcap;
-    for (uint32_t j = threadIdx.x; j < cnt; j += blockDim.x) {
-        int parent = (int)gin[64 + j];
-        if (parent < 0 || parent >= T) { atomicOr(err, 4u); continue; }
-        const int first = nodes[parent].topo.x;
-        if (first < lo || first >= hi) continue;  // another workgroup's entry
+    const int64_t lo = (int64_t)blockIdx.x * range, hi = lo + range, g = lo / from + (threadIdx.x >> lanes);
+    if (threadIdx.x == 0) s_queued = 0;
+    __syncthreads();
+    uint32_t count = 0;
+    if (g * from < hi && g * from < n) {
+        count = qin_n[g];
+        if (count > (uint32_t)from) { atomicOr(err, 4u); count = 0; }
+    }
+    for (uint32_t j = threadIdx.x & ((1u << lanes) - 1u); j < count; j += 1u << lanes) {
+        int parent = (int)qin[g * from + j];
         for (int hops = 0; parent >= 0; ++hops) {
             if (parent >= T || hops > kOctLevels) { atomicOr(err, 4u); break; }
             const OctRec r = nodes[parent];
             const int4 tp = r.topo;
-            if (!(tp.x >= lo && (int64_t)tp.x + tp.y <= hi)) {
-                const uint32_t k = atomicAdd(&gout[0], 1u);
-                if (k < qcap) gout[64 + k] = (uint32_t)parent;
-                else atomicOr(err, 4u);
+            if (qout && !(tp.x >= lo && (int64_t)tp.x + tp.y <= hi)) {
+                qout[lo + atomicAdd(&s_queued, 1u)] = (uint32_t)parent;  // one for an entry at most
                 break;
             }
             if (arrive(&flags[parent]) + 1u < (uint32_t)oct_nchild(r)) break;
@@ -632,27 +624,9 @@ __global__ __launch_bounds__(1024) void k_oct_summ_mid(OctRec *nodes, const uint
             parent = tp.w;
         }
     }
-}
-
-__global__ __launch_bounds__(1024) void k_oct_summ_global(OctRec *nodes, const uint32_t *__restrict__ misc,
-                                                          uint32_t *flags, const uint32_t *glist,
-                                                          int64_t glist_cap, float4 *quad, uint32_t *err) {
-    const int64_t T = misc[0];
-    const uint32_t cnt = glist[0] < glist_cap ? glist[0] : (uint32_t)glist_cap;
-    for (uint32_t j = threadIdx.x; j < cnt; j += blockDim.x) {
-        int parent = (int)glist[64 + j];
-        for (int hops = 0; parent >= 0; ++hops) {
-            if (parent >= T || hops > kOctLevels) { atomicOr(err, 4u); break; }
-            const OctRec r = nodes[parent];
-            if (arrive(&flags[parent]) + 1u < (uint32_t)oct_nchild(r)) break;
-            if (r.topo.z <= parent || r.topo.z + oct_nchild(r) > T || r.topo.w >= parent) {
-                atomicOr(err, 4u);
-                break;
-            }
-            oct_summ_inner(parent, r, nodes, quad);
-            parent = r.topo.w;
-        }
-    }
+    if (!qout) return;
+    __syncthreads();
+    if (threadIdx.x == 0) qout_n[blockIdx.x] = s_queued;
 }
 
 inline unsigned blocks_for(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
@@ -770,22 +744,25 @@ void launch_octree_forest_topology(int64_t n, int nsys, const float *bbox6, cons
 void launch_octree_summaries(const float4 *bodies, int64_t n, OctBuffers &ob, const int32_t *leaf_start,
                              uint32_t *err, hipStream_t s, float4 *quad) {
     if (n <= 0) return;
-    // queue layout: local -> middle at glist, middle -> global at glist + cap + 64
-    uint32_t *gmid = ob.glist + ob.cap + 64;
-    const unsigned blocks = blocks_for(n, kOctSummBodies);
-    if (!quad || blocks >= 512)
-        hipLaunchKernelGGL(k_oct_summ_local<true>, dim3(blocks), dim3(kOctSummBodies), 0, s, bodies, n, ob.nodes, leaf_start,
-                           ob.misc, ob.flags, ob.glist, ob.cap, quad, err);
-    else
-        hipLaunchKernelGGL(k_oct_summ_local<false>, dim3(blocks), dim3(kOctSummBodies), 0, s, bodies, n, ob.nodes, leaf_start,
-                           ob.misc, ob.flags, ob.glist, ob.cap, quad, err);
-    const unsigned mblocks = blocks_for(n, kOctSummMid);
-    const bool mid = mblocks >= kOctSummMidMinBlocks;
-    if (mid)
-        hipLaunchKernelGGL(k_oct_summ_mid, dim3(mblocks), dim3(1024), 0, s, ob.nodes, ob.misc, ob.flags, ob.glist, gmid,
-                           ob.cap, quad, err);
-    hipLaunchKernelGGL(k_oct_summ_global, dim3(1), dim3(1024), 0, s, ob.nodes, ob.misc, ob.flags,
-                       mid ? gmid : ob.glist, ob.cap, quad, err);
+    // two queues in turn: by body position, then the counts of the workgroups
+    const int64_t words = oct_queue_words(ob.n);
+    uint32_t *q[2] = {ob.glist, ob.glist + words};
+    int64_t from = kOctSegment;
+    hipLaunchKernelGGL(k_oct_summ_local, dim3(blocks_for(n, kOctSegment)), dim3(kOctSummThreads), 0, s, bodies, n,
+                       ob.nodes, leaf_start, ob.misc, ob.flags, q[0], q[0] + ob.n, quad, err);
+    for (int pass = 0;; ++pass) {
+        const int64_t segments = (n + from - 1) / from;
+        const bool last = segments <= kOctSummLast;
+        const int64_t range = from * (last ? kOctSummLast : kOctSummJoin);
+        int lanes = last ? 3 : 4;  // 1,024 threads on 128 or 64 segments, or on as few as there are
+        while (last && lanes < 10 && segments << (lanes + 1) <= kOctSummThreads) ++lanes;
+        uint32_t *in = q[pass & 1], *out = q[(pass + 1) & 1];
+        hipLaunchKernelGGL(k_oct_summ_queue, dim3(last ? 1u : (unsigned)((n + range - 1) / range)), dim3(kOctSummThreads),
+                           0, s, ob.nodes, ob.misc, ob.flags, n, in, in + ob.n, from, range, lanes, last ? nullptr : out,
+                           out + ob.n, quad, err);
+        if (last) break;
+        from = range;
+    }
 }
 
 }  // namespace nbg

@@ -35,7 +35,7 @@ int main(int argc, char **argv) {
     alloc(&b.key_hi, n); alloc(&b.key_lo, n); alloc(&b.lo_sorted, n);
     alloc(&b.nown, n); alloc(&b.nbase, n);
     alloc(&b.nfirst, cap); alloc(&b.ncount, cap); alloc(&b.nparent, cap); alloc(&b.nmeta, cap);
-    alloc(&b.occ, cap); alloc(&b.cb, cap); alloc(&b.flags, cap); alloc(&b.glist, 2 * (cap + 64));
+    alloc(&b.occ, cap); alloc(&b.cb, cap); alloc(&b.flags, cap); alloc(&b.glist, 2 * oct_queue_words(n));
     alloc(&b.scan_ws, oct_scan_words(n, cap));
     alloc(&b.nodes, cap); alloc(&b.centre, cap); alloc(&b.thr, 64); alloc(&b.misc, 64);
     b.cap = cap;

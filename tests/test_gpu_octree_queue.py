@@ -23,3 +23,11 @@ def test_queue_forms(nbg, orc, gpu_ctx, quad, n):
     want = np.asarray(t.accel(b.x[at], b.y[at], b.z[at]))
     assert np.array_equal(acc[at].view(np.uint32), want.view(np.uint32))
     s.close()
+
+
+@pytest.mark.parametrize("quad,n", [(False, 128 * 1024), (False, 128 * 1024 + 1), (True, 192 * 1024 + 1),
+                                    (False, 129 * 64 * 1024 + 1)])
+def test_segments(nbg, orc, gpu_ctx, quad, n):
+    """As many segments of 1,024 bodies as the last workgroup joins, one more,
+    a middle pass whose last workgroup owns one body, and two middle passes."""
+    test_queue_forms(nbg, orc, gpu_ctx, quad, n)
