@@ -49,8 +49,8 @@ void launch_fills(const FillSet &f, hipStream_t s) {
 // ------------------------------------------------------------------ bbox
 // outerBoundingBox (Physics/Summaries/SummaryType.h:73-81).  Min/max are
 // exact, so a tree-shaped reduction equals the reference's serial loop for
-// finite inputs (up to which of +0/-0 survives a tie).  The last block to
-// finish reduces the per-block partials.
+// finite inputs (up to which of +0/-0 survives a tie).  The kernel that
+// computes the keys folds the per-block partials (fold_bbox).
 // The build's first kernel: it also clears the words that the later ones
 // count in (a launch of its own for each cost 4 us at small sizes).
 __global__ __launch_bounds__(256) void k_bbox(const float *__restrict__ x, const float *__restrict__ y,
@@ -130,7 +130,7 @@ __device__ __forceinline__ K morton_key(float px, float py, float pz, const floa
 // 0: the box is folded from k_bbox's partials and stored in bbox6;
 // otherwise it is read from bbox6.
 template <typename K>
-__global__ __launch_bounds__(256) void k_morton(const float *__restrict__ x, const float *__restrict__ y,
+__global__ __launch_bounds__(kKeyThreads) void k_morton(const float *__restrict__ x, const float *__restrict__ y,
                                                 const float *__restrict__ z, int64_t n,
                                                 const float *__restrict__ partials, int blocks, float *bbox6,
                                                 K *__restrict__ keys, uint32_t *__restrict__ idx,
@@ -157,15 +157,14 @@ void launch_morton(const float *x, const float *y, const float *z, int64_t n, co
                    float *bbox6, int bits, const SortPlan &plan, void *keys, uint32_t *idx, void *keys_alt,
                    uint32_t *idx_alt, uint32_t *status, hipStream_t s) {
     if (n <= 0) return;
-    int64_t g = (n + 255) / 256;
-    if (g > 256) g = 256;  // every workgroup adds its digit counts to the histograms
+    const dim3 g(key_blocks(n)), t(key_threads(n));
     void *k = plan.from_alt ? keys_alt : keys;
     uint32_t *v = plan.from_alt ? idx_alt : idx;
     if (bits == 30)
-        hipLaunchKernelGGL(k_morton<uint32_t>, dim3((unsigned)g), dim3(256), 0, s, x, y, z, n, partials, blocks, bbox6,
+        hipLaunchKernelGGL(k_morton<uint32_t>, g, t, 0, s, x, y, z, n, partials, blocks, bbox6,
                            (uint32_t *)k, v, status, plan.passes, plan.shift);
     else
-        hipLaunchKernelGGL(k_morton<uint64_t>, dim3((unsigned)g), dim3(256), 0, s, x, y, z, n, partials, blocks, bbox6,
+        hipLaunchKernelGGL(k_morton<uint64_t>, g, t, 0, s, x, y, z, n, partials, blocks, bbox6,
                            (uint64_t *)k, v, status, plan.passes, plan.shift);
 }
 

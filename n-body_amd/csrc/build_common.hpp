@@ -13,14 +13,28 @@ namespace nbg {
 __device__ __forceinline__ float fmin_ref(float a, float b) { return (b < a) ? b : a; }
 __device__ __forceinline__ float fmax_ref(float a, float b) { return (a < b) ? b : a; }
 
+// The kernels that compute the keys take few workgroups, since each adds its
+// digit counts to the sort's histograms, and more threads in each where a
+// thread would have many bodies.  Keys phase, us, 256 workgroups of 256
+// threads at every size / this rule: octree paths, 1,000,000 bodies 56 / 36,
+// 4,000,000 199 / 92, 16,777,216 832 / 331; 63-bit codes 21 / 18, 54 / 33, 239 /
+// 90.  1,024 threads for 70,000 bodies 16 to 14, 512 workgroups for 1,000,000
+// codes 22 to 18, for 16,777,216 90 to 105.
+constexpr int kKeyThreads = 1024;
+inline int key_threads(int64_t n) { return n <= 131072 ? 256 : kKeyThreads; }
+inline unsigned key_blocks(int64_t n) {
+    const int64_t g = (n + key_threads(n) - 1) / key_threads(n), most = n < ((int64_t)1 << 22) ? 256 : 512;
+    return (unsigned)(g < most ? g : most);
+}
+
 // Second stage, at the start of the kernel that computes the keys: every
 // workgroup folds the per-block partials (the kernel boundary makes them
 // visible; no agent-scope fence, which on gfx950 is an L2 write-back +
 // invalidate) into bb, in one order, and the first one stores the box.
 __device__ __forceinline__ void fold_bbox(const float *__restrict__ partials, int blocks, float *bb, float *out6) {
-    __shared__ float s_part[4][6];
+    __shared__ float s_part[kKeyThreads / kWave][6];
     float mn[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, mx[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
-    for (int b = threadIdx.x; b < blocks; b += 256)
+    for (int b = threadIdx.x; b < blocks; b += blockDim.x)
         for (int d = 0; d < 3; ++d) {
             mn[d] = fmin_ref(mn[d], partials[b * 6 + d]);
             mx[d] = fmax_ref(mx[d], partials[b * 6 + 3 + d]);
@@ -37,7 +51,7 @@ __device__ __forceinline__ void fold_bbox(const float *__restrict__ partials, in
         for (int d = 0; d < 3; ++d) { s_part[w][d] = mn[d]; s_part[w][3 + d] = mx[d]; }
     __syncthreads();
     for (int d = 0; d < 3; ++d) { mn[d] = s_part[0][d]; mx[d] = s_part[0][3 + d]; }
-    for (int ww = 1; ww < 4; ++ww)
+    for (int ww = 1; ww < (int)blockDim.x / kWave; ++ww)
         for (int d = 0; d < 3; ++d) { mn[d] = fmin_ref(mn[d], s_part[ww][d]); mx[d] = fmax_ref(mx[d], s_part[ww][3 + d]); }
     for (int d = 0; d < 3; ++d) { bb[d] = mn[d]; bb[3 + d] = mx[d]; }
     if (blockIdx.x == 0 && threadIdx.x == 0)

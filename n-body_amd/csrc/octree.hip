@@ -217,10 +217,10 @@ __device__ __forceinline__ void oct_path(const float *bb, int levels, float px, 
     }
 }
 
-// Keys, iota payload, the sort's digit histograms of the high word and (first
+// Keys, iota payload, the sort's digit histograms of the high word and (last
 // workgroup) the opening thresholds; the box is folded from k_bbox's partials.
 template <bool LO>
-__global__ __launch_bounds__(256) void k_oct_keys(const float *__restrict__ x, const float *__restrict__ y,
+__global__ __launch_bounds__(kKeyThreads) void k_oct_keys(const float *__restrict__ x, const float *__restrict__ y,
                                                   const float *__restrict__ z, int64_t n,
                                                   const float *__restrict__ partials, int blocks, float *bbox6,
                                                   int levels, float theta, float *thr, uint64_t *khi, uint64_t *klo,
@@ -647,15 +647,14 @@ void launch_octree_keys(const float *x, const float *y, const float *z, int64_t 
                         uint32_t *idx, uint64_t *keys_alt, uint32_t *idx_alt, uint32_t *status, hipStream_t s) {
     if (n <= 0) return;
     const int levels = max_depth + 2;
-    int64_t g = (n + 255) / 256;
-    if (g > 256) g = 256;  // every workgroup adds its digit counts to the histograms
+    const dim3 g(key_blocks(n)), t(key_threads(n));
     uint64_t *k = plan.from_alt ? keys_alt : keys;
     uint32_t *v = plan.from_alt ? idx_alt : idx;
     if (levels > kOctHiLevels)
-        hipLaunchKernelGGL(k_oct_keys<true>, dim3((unsigned)g), dim3(256), 0, s, x, y, z, n, partials, blocks, bbox6,
+        hipLaunchKernelGGL(k_oct_keys<true>, g, t, 0, s, x, y, z, n, partials, blocks, bbox6,
                            levels, theta, ob.thr, k, ob.key_lo, v, status, plan.passes, plan.shift);
     else
-        hipLaunchKernelGGL(k_oct_keys<false>, dim3((unsigned)g), dim3(256), 0, s, x, y, z, n, partials, blocks, bbox6,
+        hipLaunchKernelGGL(k_oct_keys<false>, g, t, 0, s, x, y, z, n, partials, blocks, bbox6,
                            levels, theta, ob.thr, k, (uint64_t *)nullptr, v, status, plan.passes, plan.shift);
 }
 

@@ -41,7 +41,7 @@ def _params(nbg, solver, bits, leaf=16):
 
 
 @pytest.mark.parametrize("bits", [30, 63])
-@pytest.mark.parametrize("kind,n", [("cube", 1), ("cube", 2), ("cube", 1023), ("cube", 1025), ("cube", 262145),
+@pytest.mark.parametrize("kind,n", [("cube", 1), ("cube", 2), ("cube", 1023), ("cube", 1025), ("cube", 131073), ("cube", 262145), ("cube", 4194305),
                                     ("cluster", 258), ("cluster", 5000), ("cluster", 40000), ("cluster", 16386), ("cluster", 16387),
                                     ("cluster", 300001), ("escapers", 1200000), ("coincident", 3000), ("coincident", 70000),
                                     ("clusters", 5001), ("clusters", 90000), ("clusters", 1200000)])
@@ -102,3 +102,24 @@ def test_escapers_cost(nbg, gpu_ctx, solver, n):
         s.close()
     print(f"[sort] {solver} n={n} ms {ms}", flush=True)
     assert ms["escapers"] <= 12 * ms["cube"]
+
+
+def test_keys_of_large_systems(nbg, gpu_ctx):
+    """The keys of 16,777,216 bodies take 5 times as long as those of 1,048,576;
+    with 256 workgroups of 256 threads for both it was 12 times."""
+    ms = {}
+    for n in (1 << 20, 1 << 24):
+        p = _params(nbg, nbg.LINEAR_BVH, 63, leaf=32)
+        p.theta = 1.2
+        s = nbg.System(gpu_ctx, p, n)
+        s.set_state(nbg.cube(n, seed=3, side=2.0))
+        s.enable_counts(False)
+        s.enable_timing(True)
+        times = []
+        for _ in range(10):
+            s.update_accelerations()
+            times.append(s.phase_times()["keys"])
+        s.close()
+        ms[n] = min(times)
+    print(f"[sort] keys, ms {ms}", flush=True)
+    assert ms[1 << 24] <= 8 * ms[1 << 20]
