@@ -232,7 +232,7 @@ int split_of(const nbg_sys *s, int64_t nt) {
     if (s->split_req > 0) return s->split_req;
     const int64_t groups = (nt + 63) / 64;
     const bool octree = solver == NBG_BARNES_HUT || solver == NBG_BARNES_HUT_QUADRUPOLE;
-    return s->prm.sum_mode == NBG_SUM_FAST ? fast_split_waves(groups) : ordered_split_waves(groups, octree);
+    return s->prm.sum_mode == NBG_SUM_FAST ? fast_split_waves(groups) : ordered_split_waves(groups, octree, s->n);
 }
 
 // Waves per 64 targets of the system's own walk when it is split by subtrees.

@@ -181,7 +181,7 @@ int walk_tpl(const nbg_batch *b) {
 // walks), or by the number of groups, as for one system (the bits do not
 // depend on it).
 int forest_split(const nbg_batch *b) {
-    if (b->sum_mode != NBG_SUM_FAST) return ordered_split_waves(b->nwaves, is_octree_solver(b->solver));
+    if (b->sum_mode != NBG_SUM_FAST) return ordered_split_waves(b->nwaves, is_octree_solver(b->solver), b->largest);
     return b->split_req > 0 ? b->split_req : fast_split_waves(b->nwaves);
 }
 

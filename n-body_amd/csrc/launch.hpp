@@ -407,9 +407,17 @@ void launch_rows_in(const RowSet &R, int cnt, int stride, const float *words, ui
 // / 5,393; 400,000 8,911 / - / 7,426.  Linear BVH, 8 / 16 / split: 3,000 142 /
 // 118 / 478; 5,000 272 / 267 / 720; 10,000 891 / 987 / 1,026; 16,000 1,457 /
 // 2,407 / 1,595: its frames outgrow the slots.
-inline int ordered_split_waves(int64_t groups, bool octree) {
-    if (octree) return groups <= 32 ? 16 : groups <= 4096 ? 8 : 1;
-    return groups <= 80 ? 16 : groups <= 256 ? 8 : 1;
+// The recursion's time is the chain of its largest tree, `bodies`, which a
+// forest's other groups hide behind; the frames' grows with the groups.  A
+// step of octrees of 64 / 1,000 / 3,000 / 11,000 bodies, ms, recursion : 8
+// waves, at 128 groups 0.34 : 0.37, 0.90 : 0.43, 1.66 : 0.45, -; 512 0.38 :
+// 0.66, 0.94 : 0.79, 1.69 : 0.83, 3.1 : 0.9; 1,024 0.43 : 1.05, 0.97 : 1.24, 1.75
+// : 1.34, 3.2 : 1.3; 4,096 0.66 : 3.3, 1.4 : 3.8, 2.4 : 4.2, 4.3 : 4.1.  Linear
+// BVHs of 64 bodies, 128 and 256 groups 0.130 : 0.125 and 0.135 : 0.155.
+inline int64_t ordered_frames_most(bool octree) { return octree ? 4096 : 256; }
+inline int ordered_split_waves(int64_t groups, bool octree, int64_t bodies) {
+    if (groups > ordered_frames_most(octree) || groups > 64 + bodies / 2) return 1;
+    return groups <= (octree ? 32 : 80) ? 16 : 8;
 }
 
 // ORDERED split of one linear BVH of n bodies past that: waves per 64 targets
@@ -419,7 +427,7 @@ constexpr int kOrderedSplitSlots = 128;
 constexpr int64_t kOrderedSplitMaxBodies = 65536;
 inline int ordered_subtree_waves(int64_t n) {
     const int64_t groups = (n + 63) / 64;
-    if (ordered_split_waves(groups, false) > 1 || n > kOrderedSplitMaxBodies) return 1;
+    if (ordered_split_waves(groups, false, n) > 1 || n > kOrderedSplitMaxBodies) return 1;
     int k = 1;
     while (k < 16 && groups * 2 * k <= 4096) k *= 2;
     return k;

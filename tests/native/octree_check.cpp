@@ -92,7 +92,7 @@ int main(int argc, char **argv) {
     w.counts = counts;
     w.err = &err;
     const int ordered = std::atoi(argv[10]);
-    w.split = ordered ? ordered_split_waves((n + 63) / 64, true) : fast_split_waves((n + 63) / 64);
+    w.split = ordered ? ordered_split_waves((n + 63) / 64, true, n) : fast_split_waves((n + 63) / 64);
     launch_walk_oct(w, ordered, 1, nullptr);
     std::printf("err %u pp %llu np %llu\n", err, counts[0], counts[1]);
     f = std::fopen(argv[7], "wb");
