@@ -204,9 +204,10 @@ int nbg_sys_walk_stats(nbg_sys *sys, uint64_t *out4);
  * the walk offers.  Results are the same bits for every choice: FAST sums
  * each target's interactions in four fixed classes, which the waves share
  * out; ORDERED computes each opened node's result from its children's alone,
- * as the reference's recursion does.  By default a linear BVH of 16,385 to
+ * as the reference's recursion does.  ORDERED, a linear BVH of 16,385 to
  * 65,536 bodies is walked with up to 16 waves per 64 targets, which keep
- * 1,536 bytes per body of results in HBM. */
+ * 1,536 bytes per body of results in HBM; larger ones, and octrees of more
+ * than 262,144 bodies, with one. */
 int nbg_sys_set_walk_split(nbg_sys *sys, int32_t waves);
 
 /* Per-phase device time (ms) of the last force pass, measured with HIP events

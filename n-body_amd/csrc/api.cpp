@@ -229,17 +229,19 @@ bool grouped(const nbg_sys *s) {
 int split_of(const nbg_sys *s, int64_t nt) {
     const int32_t solver = s->prm.solver;
     if (solver == NBG_NAIVE || solver == NBG_IMPLICIT_FMM) return 1;
-    if (s->split_req > 0) return s->split_req;
     const int64_t groups = (nt + 63) / 64;
+    if (s->prm.sum_mode == NBG_SUM_FAST) return s->split_req > 0 ? s->split_req : fast_split_waves(groups);
     const bool octree = solver == NBG_BARNES_HUT || solver == NBG_BARNES_HUT_QUADRUPOLE;
-    return s->prm.sum_mode == NBG_SUM_FAST ? fast_split_waves(groups) : ordered_split_waves(groups, octree, s->n);
+    if (s->split_req > 0) return groups <= ordered_frames_most(octree) ? s->split_req : 1;
+    return ordered_split_waves(groups, octree, s->n);
 }
 
 // Waves per 64 targets of the system's own walk when it is split by subtrees.
 int subtree_split_of(const nbg_sys *s) {
-    if (s->prm.sum_mode != NBG_SUM_ORDERED || s->split_req > 0) return 1;
+    if (s->prm.sum_mode != NBG_SUM_ORDERED) return 1;
     if (s->prm.solver != NBG_LINEAR_BVH && s->prm.solver != NBG_LINEAR_BVH_QUADRUPOLE) return 1;
-    return ordered_subtree_waves(s->n);
+    const int k = ordered_subtree_waves(s->n);
+    return k > 1 && s->split_req > 0 ? s->split_req : k;
 }
 
 void free_split(nbg_sys *s) {

@@ -77,3 +77,30 @@ def test_small_members_are_not_framed(nbg, gpu_ctx):
         batch.close()
     print(f"[frames] {ms}", flush=True)
     assert ms["SUM_ORDERED"] <= 2.5 * ms["SUM_FAST"]
+
+
+@pytest.mark.parametrize("n", [65000, 100000])
+def test_requested_waves_past_the_frames(nbg, gpu_ctx, n):
+    """An ORDERED linear BVH past 16,384 bodies walked with the waves asked for:
+    the bits of one wave, and no slower: by subtrees 0.77 of its walk's time at
+    65,000 bodies, the same walk past 65,536; by frames, which its slots do not
+    hold, 1.06 and 1.19 times its time (without counts 1.6 and 2.1)."""
+    b = nbg.plummer(n, seed=11)
+    p = nbg.default_params()
+    p.solver, p.theta, p.leaf_size, p.eps2, p.dt = nbg.LINEAR_BVH, 0.5, 16, 1e-4, 1e-7
+    p.sum_mode = nbg.SUM_ORDERED
+    s = nbg.System(gpu_ctx, p, n)
+    s.enable_timing(True)
+    ms, acc = {}, {}
+    for k in (1, 8):
+        s.set_walk_split(k)
+        s.set_state(b)
+        times = []
+        for _ in range(4):
+            acc[k] = s.update_accelerations()
+            times.append(s.phase_times()["walk"])
+        ms[k] = min(times)
+    s.close()
+    print(f"[frames] n={n} walk ms {ms}", flush=True)
+    assert np.array_equal(acc[8].view(np.uint32), acc[1].view(np.uint32))
+    assert ms[8] <= (0.95 if n <= 65536 else 1.05) * ms[1]
