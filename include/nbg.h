@@ -353,11 +353,13 @@ int nbg_batch_use_graph(nbg_batch *b, int32_t on);
 int nbg_batch_autotune(nbg_batch *b, const int32_t *leaf_sizes, int32_t k, int32_t repeats, int32_t *best,
                        float *ms_out);
 
-/* The autotuner over leaf size x targets per lane: times every pair
- * (leaf_sizes[i], tpls[j] in {1, 2, 4}) as above and keeps the fastest pair.
- * ms_out[i * kt + j] (optional) receives each mean pass time, -1 for pairs
- * the batch does not offer (more than one target per lane exists for FAST
- * linear-BVH batches only, where it is a hint: see nbg_params).  The
+/* The autotuner over leaf size x targets per lane: gives every pair
+ * (leaf_sizes[i], tpls[j] in {1, 2, 4}) its time as above and keeps the
+ * fastest pair, the first of equal ones.  ms_out[i * kt + j] (optional)
+ * receives each mean pass time, -1 for pairs the batch does not offer (more
+ * than one target per lane exists for FAST linear-BVH batches only).  Targets
+ * per lane are a hint that the present walks do not need (nbg_params): each
+ * leaf size is timed once, and its pairs have that time.  The
  * traversal stacks need no tuning: each walk's stack holds what its trees
  * can need. */
 int nbg_batch_autotune_grid(nbg_batch *b, const int32_t *leaf_sizes, int32_t kl, const int32_t *tpls, int32_t kt,

@@ -92,8 +92,7 @@ struct nbg_batch {
     OctBuffers ob;
     int32_t *lv_tab = nullptr;
     int max_levels = 0;
-    // targets per lane asked for (the autotuner's bodies-per-wavefront
-    // choice): a hint that the present walks do not need
+    // targets per lane asked for: a hint that the present walks do not need
     int32_t tpl = 1;
     int64_t largest = 0;    // bodies of the largest member
     bool grouped = false;   // a member takes its targets in groups (kGroupMin)
@@ -772,23 +771,25 @@ int nbg_batch_autotune_grid(nbg_batch *b, const int32_t *leaf_sizes, int32_t kl,
     int32_t bl = leaf_sizes[0], bt = b->tpl;
     int r = NBG_OK;
     for (int i = 0; i < kl && r == NBG_OK; ++i) {
+        // every number of targets per lane is the same schedule: one timing
+        // serves all that are offered, and the first of them is kept
+        float ms = -1.0f;
         for (int j = 0; j < kt && r == NBG_OK; ++j) {
             if (ms_out) ms_out[i * kt + j] = -1.0f;
             b->tpl = tpls[j];
-            // a walk without a multi-target form runs one target per lane:
-            // its other candidates would time the same schedule again
             if (walk_tpl(b) != tpls[j]) continue;
-            for (Member &mm : b->sys) mm.p.leaf_size = leaf_sizes[i];
-            b->tables_dirty = true;
-            if ((r = upload_tables(b))) break;
-            enqueue_pass(b);  // warm-up
-            (void)hipEventRecord(e0, b->stream);
-            for (int t = 0; t < repeats; ++t) enqueue_pass(b);
-            (void)hipEventRecord(e1, b->stream);
-            if ((r = sync_check(b))) break;
-            float ms = 0.0f;
-            (void)hipEventElapsedTime(&ms, e0, e1);
-            ms /= (float)repeats;
+            if (ms < 0.0f) {
+                for (Member &mm : b->sys) mm.p.leaf_size = leaf_sizes[i];
+                b->tables_dirty = true;
+                if ((r = upload_tables(b))) break;
+                enqueue_pass(b);  // warm-up
+                (void)hipEventRecord(e0, b->stream);
+                for (int t = 0; t < repeats; ++t) enqueue_pass(b);
+                (void)hipEventRecord(e1, b->stream);
+                if ((r = sync_check(b))) break;
+                (void)hipEventElapsedTime(&ms, e0, e1);
+                ms /= (float)repeats;
+            }
             if (ms_out) ms_out[i * kt + j] = ms;
             if (!have || ms < best_ms) { best_ms = ms; bl = leaf_sizes[i]; bt = tpls[j]; have = true; }
         }

@@ -269,3 +269,16 @@ def test_forest_large_equals_alone(nbg, gpu_ctx, mode, solver):
         a1, _, _ = _alone(nbg, gpu_ctx, b, kw, mode, solver=solver)
         assert np.array_equal(acc.view(np.uint32), a1.view(np.uint32))
     B.close()
+
+
+def test_autotune_times_a_schedule_once(nbg, gpu_ctx):
+    """Targets per lane change no walk: a leaf size's pairs share one timing,
+    and the first of them is chosen, whatever the noise."""
+    B = nbg.Batch(gpu_ctx, 40000, 16)
+    for b, kw in _systems(nbg):
+        B.add(_params(nbg, **kw), b)
+    leaf, tpl, table = B.autotune_grid((8, 16, 32), (2, 1, 4), repeats=3)
+    for l in (8, 16, 32):
+        assert table[l, 1] == table[l, 2] == table[l, 4]
+    assert tpl == 2 and table[leaf, 2] == min(table.values())
+    B.close()
