@@ -19,7 +19,7 @@ __global__ void k_fill_u32(uint32_t *p, uint32_t v, int64_t n) {
         p[i] = v;
 }
 
-__device__ __forceinline__ void set_ranges(const FillSet &fills) {
+__device__ __forceinline__ void set_ranges(const FillRanges &fills) {
     for (int f = 0; f < fills.k; ++f) {
         uint32_t *q = fills.r[f].p;
         const uint32_t v = fills.r[f].v;
@@ -36,14 +36,19 @@ void launch_fill_u32(uint32_t *p, uint32_t v, int64_t n, hipStream_t s) {
     hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)blocks), dim3(256), 0, s, p, v, n);
 }
 
-__global__ __launch_bounds__(256) void k_fills(FillSet fills) { set_ranges(fills); }
+__global__ __launch_bounds__(256) void k_fills(FillRanges fills) { set_ranges(fills); }
+
+static void launch_more(const FillSet &f, hipStream_t s) {
+    for (const FillRanges::Range &q : f.more) launch_fill_u32(q.p, q.v, q.n, s);
+}
 
 void launch_fills(const FillSet &f, hipStream_t s) {
+    launch_more(f, s);
     int64_t most = 1;
     for (int i = 0; i < f.k; ++i) most = f.r[i].n > most ? f.r[i].n : most;
     int64_t blocks = (most + 255) / 256;
     if (blocks > 2048) blocks = 2048;
-    hipLaunchKernelGGL(k_fills, dim3((unsigned)blocks), dim3(256), 0, s, f);
+    hipLaunchKernelGGL(k_fills, dim3((unsigned)blocks), dim3(256), 0, s, static_cast<const FillRanges &>(f));
 }
 
 // ------------------------------------------------------------------ bbox
@@ -54,7 +59,7 @@ void launch_fills(const FillSet &f, hipStream_t s) {
 // The build's first kernel: it also clears the words that the later ones
 // count in (a launch of its own for each cost 4 us at small sizes).
 __global__ __launch_bounds__(256) void k_bbox(const float *__restrict__ x, const float *__restrict__ y,
-                                              const float *__restrict__ z, int64_t n, float *partials, FillSet fills) {
+                                              const float *__restrict__ z, int64_t n, float *partials, FillRanges fills) {
     set_ranges(fills);
     float mn[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, mx[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
@@ -85,12 +90,14 @@ __global__ __launch_bounds__(256) void k_bbox(const float *__restrict__ x, const
 
 int launch_bbox(const float *x, const float *y, const float *z, int64_t n, float *partials, const FillSet &fills,
                 hipStream_t s) {
+    launch_more(fills, s);
     int64_t most = n;
     for (int f = 0; f < fills.k; ++f) most = fills.r[f].n > 4 * most ? fills.r[f].n / 4 : most;
     int64_t blocks = (most + 255) / 256;
     if (blocks > kBBoxBlocks) blocks = kBBoxBlocks;
     if (blocks < 1) blocks = 1;
-    hipLaunchKernelGGL(k_bbox, dim3((unsigned)blocks), dim3(256), 0, s, x, y, z, n, partials, fills);
+    hipLaunchKernelGGL(k_bbox, dim3((unsigned)blocks), dim3(256), 0, s, x, y, z, n, partials,
+                       static_cast<const FillRanges &>(fills));
     return (int)blocks;
 }
 

@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <vector>
+
 namespace nbg {
 
 // Radix-sort geometry (onesweep): 256 threads x sort_items(n) keys per tile.
@@ -75,7 +77,7 @@ constexpr int kScanTile = kScanBlock * kScanItems;
 
 // Ranges of words that a build sets before its first use of them, in one
 // launch instead of one each.
-struct FillSet {
+struct FillRanges {  // what a kernel takes
     struct Range {
         uint32_t *p;
         int64_t n;
@@ -83,8 +85,14 @@ struct FillSet {
     };
     Range r[10];
     int k = 0;
+};
+struct FillSet : FillRanges {
+    std::vector<Range> more;  // ranges past the kernel's ten: a launch each
     void add(void *p, int64_t n, uint32_t v = 0u) {
-        if (n > 0 && k < 10) r[k++] = Range{(uint32_t *)p, n, v};
+        if (n <= 0) return;
+        const Range q{(uint32_t *)p, n, v};
+        if (k < 10) r[k++] = q;
+        else more.push_back(q);
     }
 };
 void launch_fills(const FillSet &f, hipStream_t s);

@@ -1,6 +1,7 @@
 // The last stage of the build's sort (build.hip) on the CPU.
 //   failed: indices as a radix pass leaves them that gave up its look-back
 //     (some never written): an error is reported, nothing is read out of bounds.
+//   fills: more ranges than a kernel takes are all set.
 //   runs: keys that share the sorted bits in runs on both sides of the run
 //     lengths at which the stage changes its way: the stable order.
 #include <algorithm>
@@ -89,9 +90,32 @@ static int runs() {
     return bad;
 }
 
+static int fills() {
+    int bad = 0;
+    for (int box = 0; box < 2; ++box)
+        for (int count : {1, 10, 11, 25}) {
+            std::vector<std::vector<uint32_t>> mem(count);
+            FillSet f;
+            for (int i = 0; i < count; ++i) {
+                mem[i].assign(3 + 500 * (i % 3), 0xA5A5A5A5u);
+                f.add(mem[i].data(), (int64_t)mem[i].size(), (uint32_t)i);
+            }
+            std::vector<float> x(100, 1.0f), partials(6 * kBBoxBlocks);
+            if (box) launch_bbox(x.data(), x.data(), x.data(), 100, partials.data(), f, nullptr);
+            else launch_fills(f, nullptr);
+            int wrong = 0;
+            for (int i = 0; i < count; ++i)
+                for (uint32_t v : mem[i]) wrong += v != (uint32_t)i;
+            std::printf("fills box=%d count=%d wrong %d\n", box, count, wrong);
+            bad += wrong != 0;
+        }
+    return bad;
+}
+
 int main(int argc, char **argv) {
     int bad = 0;
     if (argc > 1 && !std::strcmp(argv[1], "failed")) bad = failed();
+    if (argc > 1 && !std::strcmp(argv[1], "fills")) bad = fills();
     if (argc > 1 && !std::strcmp(argv[1], "runs")) bad = runs();
     if (bad) std::printf("%d wrong\n", bad);
     return bad != 0;

@@ -67,7 +67,7 @@ def test_frames_without_a_root(tmp_path):
     assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-4000:]
 
 
-@pytest.mark.parametrize("what", ["failed", "runs"])
+@pytest.mark.parametrize("what", ["failed", "runs", "fills"])
 def test_last_stage_of_the_sort(tmp_path, what):
     exe = _build(str(tmp_path), "sort_check.cpp", ["build"], asan=True)
     r = _run(exe, what)
