@@ -219,11 +219,6 @@ int ensure_fmm(nbg_sys *s) {
     return NBG_OK;
 }
 
-// Whether the system's walk takes its targets in compact groups (targets.hip).
-bool grouped(const nbg_sys *s) {
-    return s->n >= kGroupMin && s->prm.solver != NBG_NAIVE && s->prm.solver != NBG_IMPLICIT_FMM;
-}
-
 // Waves that share a group of targets in a walk of nt of them (1 for the
 // solvers without a tree walk): chosen by size, or as requested.
 int split_of(const nbg_sys *s, int64_t nt) {
@@ -234,6 +229,13 @@ int split_of(const nbg_sys *s, int64_t nt) {
     const bool octree = solver == NBG_BARNES_HUT || solver == NBG_BARNES_HUT_QUADRUPOLE;
     if (s->split_req > 0) return groups <= ordered_frames_most(octree) ? s->split_req : 1;
     return ordered_split_waves(groups, octree, s->n);
+}
+
+// Whether the system's walk takes its targets in compact groups (targets.hip).
+bool grouped(const nbg_sys *s) {
+    if (s->prm.solver == NBG_NAIVE || s->prm.solver == NBG_IMPLICIT_FMM) return false;
+    const bool chains = s->prm.sum_mode == NBG_SUM_ORDERED && split_of(s, s->n) == 1;
+    return s->n >= (chains ? kGroupMinChains : kGroupMin);
 }
 
 // Waves per 64 targets of the system's own walk when it is split by subtrees.

@@ -387,6 +387,12 @@ struct WalkArgs {
 // and pass, us, without / with: octree 80,000 bodies 246 / 278, 131,000 340 /
 // 360, 160,000 409 / 387; linear BVH 64,000 438 / 442, 131,000 794 / 784.
 constexpr int64_t kGroupMin = 160000;
+// The ORDERED recursion, one wave per 64 targets, gains later, when its waves
+// no longer end together; walk ms, without / with: octree 300,000 bodies 6.6 /
+// 7.4, 400,000 7.4 / 7.6, 600,000 10.9 / 10.8, 1,000,000 15.9 / 14.9; linear BVH
+// 200,000 9.9 / 10.2, 400,000 15.0 / 14.5, 600,000 20.9 / 20.2.  (By frames,
+// octree 200,000 4.9 / 4.6.)
+constexpr int64_t kGroupMinChains = 500000;
 void launch_group_targets(const float4 *bodies, const uint32_t *perm, int64_t n, float4 *out, uint32_t *out_perm,
                           hipStream_t s);
 // A forest's: systems below kGroupMin keep their order.

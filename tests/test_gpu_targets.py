@@ -57,3 +57,16 @@ def test_mixed_forest_same_bits(nbg, gpu_ctx, solver):
         s.close()
         assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), b.n
     batch.close()
+
+
+@pytest.mark.parametrize("solver,n", [("BARNES_HUT", 160001), ("LINEAR_BVH", 500001)])
+def test_every_target_once(nbg, gpu_ctx, solver, n):
+    """All bodies of a grouped ORDERED pass have the bits of a walk without
+    groups: the same points walked as passive ones, in Morton order."""
+    b = nbg.plummer(n, seed=n)
+    s = nbg.System(gpu_ctx, _params(nbg, solver, nbg.SUM_ORDERED, theta=1.0), n)
+    s.set_state(b)
+    acc = s.update_accelerations()
+    want = s.accelerations_at(b.x, b.y, b.z)
+    s.close()
+    assert np.array_equal(acc.view(np.uint32), want.view(np.uint32))
