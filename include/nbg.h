@@ -155,7 +155,7 @@ int nbg_sys_accelerations_at(nbg_sys *sys, int64_t nt, const float *tx, const fl
  * allocate (code under HIP graph capture, tight serving loops, harnesses
  * that forbid hipMalloc); it has no counterpart in the reference.  It calls
  * no hipMalloc, hipFree or allocating library routine: its scratch is one
- * static device array per GPU (about 17 MB, held until the process ends),
+ * static device array per GPU (about 19 MB, held until the process ends),
  * so at most NBG_NOALLOC_MAX_POINTS targets per call (more: NBG_ERR_ARG).
  * Every call on one GPU shares that array: calls that overlap on one GPU
  * (from several threads, on any systems of that device) race. */

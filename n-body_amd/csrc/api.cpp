@@ -590,7 +590,7 @@ PointsBuf points_carve(void *base, int64_t nt) {
 }
 
 // Scratch of nbg_sys_accelerations_at_noalloc: a file-scope device array
-// (points_layout of NBG_NOALLOC_MAX_POINTS targets, about 17 MB) that every
+// (points_layout of NBG_NOALLOC_MAX_POINTS targets, about 19 MB) that every
 // GPU the library runs on holds until the process ends.  In host code its
 // name is not a device address: nbg_ctx_create looks up each device's own
 // copy with hipGetSymbolAddress, with that device current, and host code

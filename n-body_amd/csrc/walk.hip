@@ -786,9 +786,7 @@ __device__ __forceinline__ uint64_t oct_eval_ordered(const OctRec &nd, const flo
 
 // The ORDERED octree descent from node `start` for the lanes of `smask`: the
 // node's result into r (assigned, as the reference's recursion returns it),
-// counts into cpp / cnp.  COMBINE: a child that is not a top node (with the
-// root's cut) is a frontier node: its result is taken from split_part_f
-// (slot fi, counted in visit order) instead of being evaluated.
+// counts into cpp / cnp.
 template <int MAXL, bool QUAD, bool ROWS>
 __device__ __forceinline__ void oct_ordered_descent(const WalkArgs &a, int start, uint64_t smask, float px, float py,
                                                     float pz, float G, float eps2, int *s_node, int *s_pos,
