@@ -41,9 +41,8 @@ def _params(nbg, solver, bits, leaf=16):
 
 
 @pytest.mark.parametrize("bits", [30, 63])
-@pytest.mark.parametrize("kind,n", [("cube", 1), ("cube", 2), ("cube", 1023), ("cube", 1025), ("cube", 131073), ("cube", 262145), ("cube", 4194305),
-                                    ("cluster", 258), ("cluster", 5000), ("cluster", 40000), ("cluster", 16386), ("cluster", 16387),
-                                    ("cluster", 300001), ("escapers", 1200000), ("coincident", 3000), ("coincident", 70000),
+@pytest.mark.parametrize("kind,n", [("cube", 1), ("cube", 2), ("cube", 1023), ("cube", 1025), ("cube", 262145),
+                                    ("cluster", 258), ("cluster", 5000), ("cluster", 40000), ("coincident", 3000),
                                     ("clusters", 5001), ("clusters", 90000), ("clusters", 1200000)])
 def test_linear_bvh_order(nbg, orc, gpu_ctx, kind, n, bits):
     print(f"[sort] {kind} n={n} bits={bits}", flush=True)
@@ -60,8 +59,7 @@ def test_linear_bvh_order(nbg, orc, gpu_ctx, kind, n, bits):
     assert np.array_equal(keys, want[order])
 
 
-@pytest.mark.parametrize("kind,n,leaf", [("cluster", 300, 1), ("cluster", 6000, 16), ("cluster", 20000, 16),
-                                         ("escapers", 150000, 8), ("coincident", 700, 4),
+@pytest.mark.parametrize("kind,n,leaf", [("cluster", 300, 1), ("cluster", 6000, 16), ("coincident", 700, 4),
                                          ("clusters", 9000, 8), ("cube", 257, 1)])
 def test_octree_bits(nbg, orc, gpu_ctx, kind, n, leaf):
     print(f"[sort] octree {kind} n={n} leaf={leaf}", flush=True)
@@ -76,6 +74,18 @@ def test_octree_bits(nbg, orc, gpu_ctx, kind, n, leaf):
     assert np.array_equal(acc.view(np.uint32), want.view(np.uint32))
     assert s.counts() == (int(pp.sum()), int(npc.sum()))
     s.close()
+
+
+@pytest.mark.parametrize("bits", [30, 63])
+@pytest.mark.parametrize("kind,n", [("cube", 131073), ("cube", 4194305), ("cluster", 16386), ("cluster", 16387),
+                                    ("cluster", 300001), ("escapers", 1200000), ("coincident", 70000)])
+def test_long_runs_order(nbg, orc, gpu_ctx, kind, n, bits):
+    test_linear_bvh_order(nbg, orc, gpu_ctx, kind, n, bits)
+
+
+@pytest.mark.parametrize("kind,n,leaf", [("cluster", 20000, 16), ("escapers", 150000, 8)])
+def test_long_runs_octree(nbg, orc, gpu_ctx, kind, n, leaf):
+    test_octree_bits(nbg, orc, gpu_ctx, kind, n, leaf)
 
 
 @pytest.mark.parametrize("solver", ["LINEAR_BVH", "BARNES_HUT"])
