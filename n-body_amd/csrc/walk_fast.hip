@@ -31,9 +31,10 @@
 // of them, 15 with masks.  Measured against that walk, ms a pass: linear BVH
 // 7.71 -> 5.20, octree 3.74 -> 2.05 (1,048,576 bodies), quadrupole linear
 // BVH 2.51 -> 1.90 (500,000), octree 2.58 -> 1.54 (300,007, theta 0.41),
-// linear BVH of 10,000 bodies 0.41 -> 0.14.  Bound by VALU issue (linear BVH:
-// 48,200 instructions a wave and 65,536 waves are 5.2 ms at 2.3 GHz on 1,024
-// SIMDs), of which listing is 45 %; half the targets a wave would double it.
+// linear BVH of 10,000 bodies 0.41 -> 0.14.  Bound by VALU issue (linear BVH,
+// targets in compact groups: 43,100 instructions a wave and 65,536 waves are
+// 4.6 ms at 2.4 GHz on 1,024 SIMDs), of which the pairs' own are 35 %; half
+// the targets a wave would double the listing.
 //
 // Sums: the 64 sources of a list are four classes of 16; each class has its
 // own FP32 partial per lane (at most 32 terms, then added to FP64), and the
