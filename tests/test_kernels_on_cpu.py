@@ -111,3 +111,14 @@ def test_fast_walk_in_bounds(octree_exe, tmp_path, nbg, orc, n, leaf, same):
 def octree_exe(tmp_path_factory):
     return _build(str(tmp_path_factory.mktemp("octree")), "octree_check.cpp", ["build", "octree", "walk", "walk_fast"],
                   asan=True)
+
+
+def test_forest_order_of_workgroups(tmp_path):
+    """Members of 16,384 bodies are eight runs of 32 workgroups each: with run x
+    of eight always on XCD x, every member's dense eighth was on one XCD."""
+    exe = _build(str(tmp_path), "turns_check.cpp", [], False)
+    rows = [r.split() for r in subprocess.run([exe], check=True, capture_output=True, text=True).stdout.splitlines()]
+    assert len(rows) == 40
+    # most of one eighth of all members that is on one XCD, 1: shared evenly, 8: all of it
+    uneven = [r for r in rows if int(r[0]) >= 64 and float(r[2]) > 1.3]
+    assert not uneven, uneven
